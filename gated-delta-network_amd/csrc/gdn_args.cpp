@@ -199,10 +199,30 @@ int check_prefill_args(const gdn_bf16 *q, const gdn_bf16 *k, const gdn_bf16 *v, 
   return GDN_OK;
 }
 
+// Whether the chunks go through the fused scan (gdn_scan.hip) or the
+// operand-form pipeline: the scan, except for at most 8 (sequence, v-head)
+// groups of a middling chain, too short to be cut (segment_length) and long
+// enough for the pipeline's shorter step to pay for its third launch (us,
+// operand forms / scan: 1x640 28.2 / 26.6, 1x768 29.4 / 29.7, 1x1024 30.8 /
+// 35.4, 1x2048 39.9 / 40.0, 1x2560 49.0 / 44.5; 2x1024 38.2 / 37.6; with two
+// v-heads 1x4096 47.1 / 50.1, 2x1024 33.8 / 36.6, 2x2048 45.7 / 41.0).
+static bool scan_wins(int nt, int N, const Heads &H) {
+  const long long mean = (static_cast<long long>(nt) + N - 1) / N;
+  const long long groups = static_cast<long long>(N) * H.v;
+  return groups > 8 || mean <= 11 || mean >= (groups <= 2 ? 80 : 33);
+}
+
 int plan_prefill(int T, int N, const Heads &H, const PrefillLayout &L, int variant, int rec_max,
                  int rec_variant, int block_variant, const char *what, PrefillPlan &P) {
   P = PrefillPlan{};
   P.seq_variant = rec_variant;
+  P.scan = variant == -1 && rec_max == -1 && L.nt_max > 0 && scan_wins(L.nt_max, N, H);
+  // Cutting long sequences: for at most 64 (one lane each), when even the one
+  // that takes every token but one of each other could be worth it.
+  if (N <= 64 && L.nt_max - (N - 1) >= kScanCutMin) {
+    const int most = (L.nt_max - 1) / kMinSegment;
+    P.scan_more = 2 * kNumCus / (4 * H.v) < most ? 2 * kNumCus / (4 * H.v) : most;
+  }
   const float fT = static_cast<float>(T), fhv = static_cast<float>(H.v);
   if (rec_max >= 0) {
     P.sequential = rec_max >= T;
@@ -224,8 +244,10 @@ int plan_prefill(int T, int N, const Heads &H, const PrefillLayout &L, int varia
       // sequence ~10x faster than the chunks'): the device gets the choice
       // only if the sequential path wins there by more than the choice costs.
       const float fN = static_cast<float>(N);
-      const float chunks_eq = cost_by_chunks(mean, fN * ceilf(mean / kChunk), fhv, fN);
-      if (seq_lo + kDeviceChoiceCost < chunks_eq) P.choose = blocks ? 3 : 2;
+      const float nt_eq = fN * ceilf(mean / kChunk);
+      if (P.scan ? seq_lo < cost_by_scan(mean, nt_eq, fhv, fN)
+                 : seq_lo + kDeviceChoiceCost < cost_by_chunks(mean, nt_eq, fhv, fN))
+        P.choose = blocks ? 3 : 2;
     }
   }
   if (P.sequential) return GDN_OK;

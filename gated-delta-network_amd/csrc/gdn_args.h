@@ -116,6 +116,9 @@ constexpr int kRecurrentMaxLen = 96;
 // chunks).
 constexpr int kSplitMinChunks = 9;
 
+// Chunks of the shortest sequence that the fused scan may cut.
+constexpr int kScanCutMin = 20;
+
 // Compute units of the target (MI355X: 256).  The WY intra kernel runs each
 // (chunk, v-head) as two workgroups (its w and u halves) while that leaves
 // at most kIntraSplitPerCu workgroups per CU: a batch too small to fill the
@@ -138,6 +141,9 @@ struct PrefillPlan {
                     // (by rec_max / token vs chunk costs / block vs chunk costs)
   bool single;      // one sequence without a chunk table (bounds read on the device)
   int form;         // per-chunk operands: 0 WY, 1 T, -1 the index kernel's rule
+  bool scan;        // the chunks through the fused scan (gdn_scan.hip) instead of the
+                    // operand-form pipeline the fields below describe
+  int scan_more;    // most segments beyond the sequences' first ones (0: none is cut)
   int split_nt0;    // two-segment scan: first chunk of the second segment; 0 none
   bool intra_split; // WY intra kernel as two workgroups per (chunk, v-head)
   bool loop;        // the state kernel loops over its units in a capped grid

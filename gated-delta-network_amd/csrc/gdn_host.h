@@ -40,6 +40,14 @@ int block_launch(const uint16_t *q, const uint16_t *k, const uint16_t *v, const 
                  int *status, const Heads &H, float scale, uint16_t *out, float *new_state,
                  hipStream_t stream, const char *what);
 
+// The chunked prefill with the output fused into the recurrence
+// (gdn_scan.hip), after the index launch if the plan has one.
+int scan_launch(const uint16_t *q, const uint16_t *k, const uint16_t *v, const float *state,
+                const float *A_log, const uint16_t *a, const float *dt_bias, const uint16_t *b,
+                const void *cu, int cu64, int N, int T, const Heads &H, const PrefillLayout &L,
+                const PrefillPlan &P, float scale, uint16_t *out, float *new_state, char *ws,
+                hipStream_t stream, const char *what);
+
 // One decode step (gdn_decode.hip) with head layout H; variant as in
 // gdn_decode_fwd_variant.  Validates its arguments; messages start with `what`.
 int decode_launch(const gdn_bf16 *q, const gdn_bf16 *k, const gdn_bf16 *v, const float *state,
