@@ -219,7 +219,7 @@ int plan_prefill(int T, int N, const Heads &H, const PrefillLayout &L, int varia
   P.scan = variant == -1 && rec_max == -1 && L.nt_max > 0 && scan_wins(L.nt_max, N, H);
   // Cutting long sequences: for at most 64 (one lane each), when even the one
   // that takes every token but one of each other could be worth it.
-  if (N <= 64 && L.nt_max - (N - 1) >= kScanCutMin) {
+  if (P.scan && N <= 64 && L.nt_max - (N - 1) >= kScanCutMin) {
     const int most = (L.nt_max - 1) / kMinSegment;
     P.scan_more = 2 * kNumCus / (4 * H.v) < most ? 2 * kNumCus / (4 * H.v) : most;
   }
@@ -244,10 +244,8 @@ int plan_prefill(int T, int N, const Heads &H, const PrefillLayout &L, int varia
       // sequence ~10x faster than the chunks'): the device gets the choice
       // only if the sequential path wins there by more than the choice costs.
       const float fN = static_cast<float>(N);
-      const float nt_eq = fN * ceilf(mean / kChunk);
-      if (P.scan ? seq_lo < cost_by_scan(mean, nt_eq, fhv, fN)
-                 : seq_lo + kDeviceChoiceCost < cost_by_chunks(mean, nt_eq, fhv, fN))
-        P.choose = blocks ? 3 : 2;
+      const float chunks_eq = cost_by_chunks(mean, fN * ceilf(mean / kChunk), fhv, fN);
+      if (seq_lo + kDeviceChoiceCost < chunks_eq) P.choose = blocks ? 3 : 2;
     }
   }
   if (P.sequential) return GDN_OK;

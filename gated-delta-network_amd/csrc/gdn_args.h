@@ -142,7 +142,10 @@ struct PrefillPlan {
   bool single;      // one sequence without a chunk table (bounds read on the device)
   int form;         // per-chunk operands: 0 WY, 1 T, -1 the index kernel's rule
   bool scan;        // the chunks through the fused scan (gdn_scan.hip) instead of the
-                    // operand-form pipeline the fields below describe
+                    // operand-form pipeline the fields below describe.  The choice
+                    // between sequential and chunks stays the operand forms': the
+                    // sequential kernels are the more precise ones, so no batch
+                    // leaves them for the scan's sake
   int scan_more;    // most segments beyond the sequences' first ones (0: none is cut)
   int split_nt0;    // two-segment scan: first chunk of the second segment; 0 none
   bool intra_split; // WY intra kernel as two workgroups per (chunk, v-head)

@@ -43,8 +43,6 @@ __device__ __forceinline__ bool device_picks_sequential(int choose, int rec_max,
   const float by_seq = choose == 2 ? cost_by_token(L, static_cast<float>(T), fhv, g)
                                    : cost_by_block(L, g);
   const float fnt = static_cast<float>(chunks);
-  if (form == kFormScan)
-    return by_seq + kSeqChoiceMargin <= cost_by_scan(L, fnt, fhv, static_cast<float>(N));
   const bool t = form == 1 ||
                  (form != 0 && t_form_wins(fnt, ceilf(L / kChunk), state_units(static_cast<float>(N), fhv)));
   return by_seq + kSeqChoiceMargin <= cost_by_chunks_form(L, fnt, fhv, static_cast<float>(N), t);
@@ -190,7 +188,7 @@ __device__ __forceinline__ SelfIndexed self_index(char *smem, const SelfIndex &s
       si.offsets[N + 1] = sequential ? 1 : 0;
       si.offsets[N + 2] = form;
     }
-    if (si.form == kFormScan && si.max_more > 0 && tid < 64) {  // (N <= 64)
+    if (si.max_more > 0 && tid < 64) {  // (N <= 64)
       const int seg = segment_length(n, si.max_more, hv);
       if (tid == 0) si.offsets[N + 2] = seg;
     }

@@ -86,15 +86,6 @@ __host__ __device__ inline float cost_by_chunks(float L, float nt, float hv, flo
                              t_form_wins(nt, ceilf(L / 64.0f), state_units(N, hv)));
 }
 
-// The fused scan (gdn_scan.hip), fitted to 100 equal-length batches (N = 1..128,
-// L = 32..8192; within 10 % where the sequential paths compete): its launches
-// (an idle one, 3.5 us, included), the state's traffic per group, and the
-// larger of the work per (chunk, v-head) and the longest sequence's chain.
-__host__ __device__ inline float cost_by_scan(float L, float nt, float hv, float N) {
-  const float u = nt * hv;
-  return 16.0f + 0.038f * N * hv + fmaxf(0.030f * u, 1.65f * ceilf(L / 64.0f) + 0.006f * u);
-}
-
 // What a path choice made on the device costs (graph replay, MI355X): the
 // index kernel and the chunk kernels returning at once when the sequential
 // path wins (~9 us over the sequential kernel alone), the sequential kernel
@@ -115,9 +106,7 @@ constexpr float kSeqChoiceMargin = 4.0f;
 constexpr int kSelfIndexMax = 256;
 constexpr long long kSelfIndexMaxGrid = 2560;
 
-// Value of the form argument of the index code for the fused scan; its
-// shortest segment in chunks.
-constexpr int kFormScan = 2;
+// Shortest segment of the fused scan (gdn_scan.hip), in chunks.
 constexpr int kMinSegment = 4;
 
 // First chunk of the second segment of a two-segment scan over nt chunks.

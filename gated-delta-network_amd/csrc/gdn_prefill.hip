@@ -143,7 +143,7 @@ __global__ __launch_bounds__(1024) void prefill_index_kernel(const void *cu, int
       s_eos[tid] = eos;
     }
     most_chunks = n > most_chunks ? n : most_chunks;
-    if (form == kFormScan && max_more > 0 && tid < 64) {  // (N <= 64: one tile)
+    if (max_more > 0 && tid < 64) {  // (N <= 64: one tile)
       const int seg = segment_length(n, max_more, hv);
       if (tid == 0) offsets[N + 2] = seg;
     }
@@ -189,7 +189,7 @@ __global__ __launch_bounds__(1024) void prefill_index_kernel(const void *cu, int
   const int nt = static_cast<int>(carry < nt_max ? carry : nt_max);
   if (tid == 0) {
     offsets[N] = nt;
-    if (form != kFormScan || max_more == 0)
+    if (max_more == 0)
       offsets[N + 2] = (form == 0 || form == 1)
                          ? form
                          : (t_form_wins(static_cast<float>(nt), static_cast<float>(s_most_chunks),
@@ -2245,8 +2245,8 @@ static int prefill_launch(const gdn_bf16 *q, const gdn_bf16 *k, const gdn_bf16 *
   // (P.self_index), launched first.
   if (!P.single && !P.self_index) {
     hipLaunchKernelGGL(prefill_index_kernel, dim3(1), dim3(1024), 0, stream, cu_seqlens, cu64, N, T,
-                       L.nt_max, P.choose, rec_max, H.v, P.scan ? kFormScan : P.form,
-                       P.scan ? P.scan_more : 0, chunks, offsets, status);
+                       L.nt_max, P.choose, rec_max, H.v, P.form,
+                       P.scan_more, chunks, offsets, status);
     if ((rc = check_launch(what))) return rc;
   }
   auto sequential_kernel = [&]() {

@@ -976,7 +976,7 @@ int scan_launch(const uint16_t *q, const uint16_t *k, const uint16_t *v, const f
   int *status = reinterpret_cast<int *>(ws + L.status);
   char *rec = ws + L.w;
   const OneSeq one{P.single ? cu : nullptr, cu64, T};
-  const SelfIndex si{P.self_index ? cu : nullptr, cu64, N, T, P.choose, -1, kFormScan,
+  const SelfIndex si{P.self_index ? cu : nullptr, cu64, N, T, P.choose, -1, P.form,
                      chunks, offsets, status, nullptr, 0, P.scan_more};
   hipLaunchKernelGGL(scan_intra_kernel, dim3(static_cast<unsigned>(chunk_head_grid(L.nt_max, H))),
                      dim3(256), 0, stream, q, k, A_log, a, dt_bias, b, chunks, one, L.nt_max, H, si,
