@@ -85,6 +85,29 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
     return lib
 
 
+_native = None
+_native_tried = False
+
+
+def native():
+    """The native entry of ordinary calls (csrc/gdn_torch.cpp), bound to the
+    loaded library, or None where the extension is not built (a tree that holds
+    the library alone): the Python path then makes the same C ABI calls."""
+    global _native, _native_tried
+    if not _native_tried:
+        lib = load()
+        try:
+            from . import _native as module
+        except ImportError:
+            module = None
+        if module is not None:
+            module.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in (
+                "gdn_decode_fwd", "gdn_decode_multi_fwd", "gdn_decode_fwd_heads", "gdn_prefill_fwd",
+                "gdn_prefill_fwd_heads", "gdn_prefill_workspace_bytes_heads")))
+        _native, _native_tried = module, True
+    return _native
+
+
 def last_error() -> str:
     return load().gdn_last_error().decode(errors="replace")
 

@@ -73,6 +73,13 @@ def kernel(q, k, v, state, A_log, a, dt_bias, b, scale, output, new_state, *, va
     T>1: 0..9 token by token, 10 the 16-token block kernel); the default is
     the built-in one.
     """
+    fast = _lib.native()
+    if fast is not None and variant == -1:
+        rc = fast.decode(q, k, v, state, A_log, a, dt_bias, b, scale, output, new_state)
+        if rc == 0:
+            return
+        if rc < 0:
+            _lib.check(rc, "gdn_decode_fwd")
     lib = _lib.load()
     four = isinstance(q, torch.Tensor) and q.dim() == 4
     B = q.shape[0] if four else -1

@@ -86,6 +86,11 @@ def _workspace(dev: torch.device, stream: int, nbytes: int) -> torch.Tensor:
         return entry[0]
 
 
+def _cached(index: int, stream: int, nbytes: int) -> torch.Tensor:
+    """_workspace for the native entry: the device by its index."""
+    return _workspace(torch.device("cuda", index), stream, nbytes)
+
+
 def release_workspaces() -> int:
     """Drops the cached per-stream workspaces that no captured graph can
     write (torch's caching allocator then owns their memory again); a cached
@@ -194,6 +199,14 @@ def kernel(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output, new_
     ``recurrent_variant``: the sequential kernel (gdn_prefill_fwd_tuned):
     0..9 a token-by-token row tiling, 10 the 16-token block kernel.
     """
+    fast = _lib.native()
+    if fast is not None and variant == recurrent_max_len == recurrent_variant == -1:
+        rc = fast.prefill(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output, new_state,
+                          workspace, _cached)
+        if rc == 0:
+            return
+        if rc < 0:
+            _lib.check(rc, "gdn_prefill_fwd")
     lib = _lib.load()
     T, N, dev, heads = _validate(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, output,
                                  new_state)
