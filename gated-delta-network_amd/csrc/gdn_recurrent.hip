@@ -22,9 +22,20 @@
 // 4c..4c+3 and 64+4c..64+4c+3), so the two row dot products per token are 8
 // FMAs and 4 DPP adds.  A workgroup of WAVES waves owns 4*WAVES*PASSES rows.
 // Per token each lane loads its 8 columns of k and q (two 8-byte loads each)
-// and one bf16 of v per pass, 2-8 tokens ahead of use (a register ring); the
-// gating of a ring turn's tokens is computed at once, one token per lane, and
-// read back with readlane.
+// and v, 2-8 tokens ahead of use (a register ring); the gating of a ring turn's
+// tokens is computed at once, one token per lane, and read back with readlane.
+//
+// What bounds it: the state's one read and one write when the rows are short
+// (B=64 T=4: 70 MB), and then what a token's step issues beside them.
+// From eight passes on (kPacked) v and o take one memory instruction a token,
+// lane j of a row group carrying the row of pass j mod PASSES, instead of one
+// a pass: a token's memory instructions fall from 4 + 2 PASSES to 6 (us per
+// step, B=64 T=2 / 3 / 4, 32 rows a wave: 12.2 / 14.4 / 16.1 -> 11.6 / 14.1 /
+// 15.5; B=128, 64 rows: 21.9 / 25.4 / 28.4 -> 20.8 / 23.4 / 26.6).  With four
+// passes it gained nothing (B=64 T=2 13.6 -> 14.3); with eight, a ring of four
+// tokens instead of two lost once two waves a SIMD no longer held the launch
+// (B=128 T=4 27.3 -> 30.2), and registers held to four waves a SIMD cost more
+// (B=64 T=4 15.5 -> 19.1).
 #include "gdn_device.h"
 #include "gdn_host.h"
 
@@ -32,8 +43,9 @@ namespace gdn {
 
 template <int PASSES>
 struct TokenIn {
+  static constexpr bool kPacked = PASSES >= 8;
   u16x4 k0, k1, q0, q1;
-  uint16_t v[PASSES];
+  uint16_t v[kPacked ? 1 : PASSES];
 };
 
 template <int WAVES, int PASSES>
@@ -54,6 +66,8 @@ __global__ __launch_bounds__(64 * WAVES) void recurrent_kernel(
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c4 = 4 * (lane & 15);
   const int row0 = tile * kRows + wave * 4 * PASSES + (lane >> 4);  // pass p: row0 + 4p
+  static_assert((PASSES & (PASSES - 1)) == 0 && PASSES <= 16, "one lane of a group per pass");
+  const int jl = lane & (PASSES - 1);  // the pass whose v and o this lane carries
 
   // The path flag and the sequence's bounds, loaded together (one wait for
   // both), before the state loads, which do not depend on them.
@@ -112,13 +126,17 @@ __global__ __launch_bounds__(64 * WAVES) void recurrent_kernel(
       x.q0 = *reinterpret_cast<const u16x4 *>(qp);
       x.q1 = *reinterpret_cast<const u16x4 *>(qp + 64);
       const uint16_t *vp = v + (tok * H.v + h) * kDV + row0;
+      if constexpr (TokenIn<PASSES>::kPacked) {
+        x.v[0] = vp[4 * jl];
+      } else {
 #pragma unroll
-      for (int p = 0; p < PASSES; ++p) x.v[p] = vp[4 * p];
+        for (int p = 0; p < PASSES; ++p) x.v[p] = vp[4 * p];
+      }
     };
 
     // One token: x holds its k, q, v; (g, beta) its gating.  Every lane of a
-    // row group holds the row's o, so all 16 store the same two bytes (one
-    // coalesced write) and no lane needs a branch.
+    // row group holds the row's o, so all 16 store the same two bytes, or
+    // those of pass jl (one coalesced write), and no lane needs a branch.
     auto step = [&](const TokenIn<PASSES> &x, int t, float g, float beta) {
       float kf[8], qf[8];
 #pragma unroll
@@ -132,6 +150,8 @@ __global__ __launch_bounds__(64 * WAVES) void recurrent_kernel(
 #pragma unroll
       for (int e = 0; e < 8; ++e) pkq = fmaf(kf[e], qf[e], pkq);
       const float kq = row16_sum(pkq);
+      float vl = 0.f, ov = 0.f;  // this lane's pass jl of v and o
+      if constexpr (TokenIn<PASSES>::kPacked) vl = bf16_to_f32(x.v[0]);
       uint16_t *op = out + ((static_cast<size_t>(bos) + t) * H.v + h) * kDV + row0;
 #pragma unroll
       for (int p = 0; p < PASSES; ++p) {
@@ -145,15 +165,24 @@ __global__ __launch_bounds__(64 * WAVES) void recurrent_kernel(
         }
         const float sk = row16_sum(sk0 + sk1);
         const float sq = row16_sum(sq0 + sq1);
-        const float vn = beta * (bf16_to_f32(x.v[p]) - g * sk);
+        float vp;
+        if constexpr (TokenIn<PASSES>::kPacked)
+          vp = row_bcast16(vl, p);
+        else
+          vp = bf16_to_f32(x.v[p]);
+        const float vn = beta * (vp - g * sk);
         const float o = scale * fmaf(g, sq, vn * kq);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           Sa[p][e] = fmaf(vn, kf[e], g * Sa[p][e]);
           Sb[p][e] = fmaf(vn, kf[4 + e], g * Sb[p][e]);
         }
-        op[4 * p] = f32_to_bf16(o);
+        if constexpr (TokenIn<PASSES>::kPacked)
+          ov = jl == p ? o : ov;
+        else
+          op[4 * p] = f32_to_bf16(o);
       }
+      if constexpr (TokenIn<PASSES>::kPacked) op[4 * jl] = f32_to_bf16(ov);
     };
 
     // Everything is loaded ahead of use by unconditional loads (indices past
@@ -251,16 +280,26 @@ void launch_rec(long long groups, hipStream_t stream, const uint16_t *q, const u
 int recurrent_num_variants() { return kNumRecVariants + 1; }
 int recurrent_block_variant() { return kNumRecVariants; }
 
-// Built-in tiling from a sweep on MI355X (every tiling, B = 1..256 rows of
-// T = 2, 4, 8 tokens, graph replay over rotating states): few (sequence,
-// head) groups -> the smallest row blocks (the serial token loop is spread
-// over the most waves); more -> one wave streaming 8..32 rows (within ~5 % of
-// the best tiling everywhere; 64-row four-wave blocks, the earlier choice for
-// more than 128 groups, were up to 14 % slower at B = 64..256).
-int recurrent_default_variant(long long groups) {
+// Built-in tiling from sweeps on MI355X (every tiling, B = 1..512 rows of
+// T = 2..6 tokens with 8 v-heads, graph replay over rotating states): few
+// (sequence, head) groups -> the smallest row blocks (the serial token loop is
+// spread over the most waves); more -> one wave streaming 8..64 rows.
+// A wave's time grows with its rows times the tokens, so the smaller rows win
+// until a launch of them no longer fits the chip at once: the times jump there,
+// and the next larger block takes over.
+// us per step, 16 / 32 rows: B=40 (320 groups) T=2 9.3 / 10.2, T=4 11.5 / 13.9;
+// B=44 T=2 10.3 / 10.5; B=48 11.1 / 10.7, T=3 11.0 / 12.7; B=52 (416) T=3
+// 12.3 / 13.3, T=4 14.0 / 14.9; B=56 T=4 15.3 / 15.2.  32 / 64 rows: B=96 (768)
+// T=2 17.9 / 18.8, T=4 20.1 / 24.3; B=104 21.3 / 19.7, 24.4 / 24.6; B=128
+// 24.0 / 20.8, 27.7 / 26.6, T=5 29.7 / 30.5; B=136 26.6 / 27.5.
+// `tokens`: mean tokens of a sequence.  One-token sequences (prefill only;
+// decode has its own kernel) are outside that sweep and keep the lines of an
+// earlier one.
+int recurrent_default_variant(long long groups, long long tokens) {
   if (groups <= 32) return 0;     // 4 rows, 1 wave
   if (groups <= 64) return 3;     // 8 rows, 1 wave
-  if (groups <= 256) return 6;    // 16 rows, 1 wave
+  if (groups <= (tokens >= 3 ? 416 : tokens == 2 ? 352 : 256)) return 6;  // 16 rows, 1 wave
+  if (groups > 768 && groups <= 1024 && tokens >= 2 && tokens <= 4) return 9;  // 64 rows, 1 wave
   if (groups <= 1024) return 8;   // 32 rows, 1 wave
   return 6;                       // 16 rows, 1 wave
 }
@@ -272,7 +311,7 @@ int recurrent_launch(const uint16_t *q, const uint16_t *k, const uint16_t *v, co
                      float scale, uint16_t *out, float *new_state, hipStream_t stream,
                      int variant, const char *what) {
   const long long groups = static_cast<long long>(num_seqs) * H.v;
-  if (variant < 0) variant = recurrent_default_variant(groups);
+  if (variant < 0) variant = recurrent_default_variant(groups, num_seqs > 0 ? T / num_seqs : 0);
   if (variant == kNumRecVariants)
     return block_launch(q, k, v, state, A_log, a, dt_bias, b, cu, cu64, num_seqs, T, fixed_len,
                         enable, status, H, scale, out, new_state, stream, what);

@@ -293,6 +293,21 @@ def test_multi_token_decode_tilings_are_identical(cuda_device):
     _check(ref_o.reshape(B * T, 8, 128), ref_s, inp, tight=True)
 
 
+# Both sides of the lines between 16, 32 and 64 rows a wave (44, 52, 96 and 128
+# rows of 8 v-heads), token counts around the two-token ring of the larger ones.
+@pytest.mark.parametrize("B, T", [(44, 2), (45, 2), (52, 3), (53, 3), (96, 3), (97, 2), (97, 3),
+                                  (128, 4), (128, 5), (129, 2)])
+def test_multi_token_decode_tiling_lines(cuda_device, B, T):
+    inp, dec = _multi_inputs(B, T, seed=35 + B + T)
+    d = _to_dev(dec, cuda_device)
+    out, ns = _decode_multi(d, B, T, cuda_device)
+    # the same sums in the same order in every tiling: equal bits
+    for var in (0, 8, 9):
+        o, s = _decode_multi(d, B, T, cuda_device, variant=var)
+        assert torch.equal(o, out) and torch.equal(s, ns), f"tiling {var}"
+    _check(out.reshape(B * T, 8, 128), ns, inp, tight=True)
+
+
 # ---------------------------------------------------------------------------
 # the 16-token block kernel (gdn_block.hip; recurrent variant BLOCK)
 # ---------------------------------------------------------------------------
