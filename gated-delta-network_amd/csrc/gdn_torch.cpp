@@ -212,4 +212,13 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", "ordinary calls of the G
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__native() { return PyModule_Create(&module); }
+// torch_version: the torch this was compiled against.  Tensors are unpacked by
+// that version's layout, so gdn_amd._lib binds the module under no other.
+PyMODINIT_FUNC PyInit__native() {
+  PyObject *m = PyModule_Create(&module);
+  if (m != nullptr && PyModule_AddStringConstant(m, "torch_version", GDN_TORCH_VERSION) < 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

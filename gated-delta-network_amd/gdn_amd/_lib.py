@@ -9,7 +9,9 @@ anything but the HIP kernels.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
 import os
+import warnings
 
 LIB_NAME = "libgdn_amd.so"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
@@ -89,17 +91,38 @@ _native = None
 _native_tried = False
 
 
+def _native_file() -> str | None:
+    """The built extension beside this file, or None."""
+    here = os.path.dirname(LIB_PATH)
+    files = [os.path.join(here, "_native" + s) for s in importlib.machinery.EXTENSION_SUFFIXES]
+    return next((f for f in files if os.path.exists(f)), None)
+
+
 def native():
     """The native entry of ordinary calls (csrc/gdn_torch.cpp), bound to the
     loaded library, or None where the extension is not built (a tree that holds
-    the library alone): the Python path then makes the same C ABI calls."""
+    the library alone): the Python path then makes the same C ABI calls.  One
+    that is there but does not load, or was built against another torch (whose
+    tensors it would misread), is not used either, with a warning."""
     global _native, _native_tried
     if not _native_tried:
+        import torch  # (the library alone needs none)
         lib = load()
+        module = None
         try:
             from . import _native as module
-        except ImportError:
-            module = None
+        except ImportError as e:
+            if _native_file() is not None:
+                warnings.warn(f"{_native_file()} does not load ({e}): calls take the Python path",
+                              RuntimeWarning, stacklevel=2)
+        if module is not None:
+            built = getattr(module, "torch_version", None)
+            if built != torch.__version__:
+                warnings.warn(f"gdn_amd._native was built against torch {built}, this is "
+                              f"{torch.__version__}: calls take the Python path (rebuild with "
+                              "`make -C gated-delta-network_amd/csrc -B native`)",
+                              RuntimeWarning, stacklevel=2)
+                module = None
         if module is not None:
             module.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in (
                 "gdn_decode_fwd", "gdn_decode_multi_fwd", "gdn_decode_fwd_heads", "gdn_prefill_fwd",

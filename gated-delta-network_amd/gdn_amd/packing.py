@@ -240,7 +240,9 @@ def load_entry(doc: dict, dest):
 
 def ensure_library(jobs: int = 8) -> str:
     """Build libgdn_amd.so from the sources beside this package if it is not
-    there yet (one builder at a time, under a file lock); return its path."""
+    there yet (one builder at a time, under a file lock); return its path.  The
+    native entry of ordinary calls is built with it where this interpreter's
+    headers allow; without it, calls take the Python path (_lib.native)."""
     lib = _lib.LIB_PATH
     if os.path.exists(lib):
         return lib
@@ -248,11 +250,12 @@ def ensure_library(jobs: int = 8) -> str:
     with open(csrc / ".build.lock", "w") as lock:
         fcntl.flock(lock, fcntl.LOCK_EX)
         if not os.path.exists(lib):
-            r = subprocess.run(["make", "-C", str(csrc), f"-j{int(jobs)}"],
-                               capture_output=True, text=True)
+            make = ["make", "-C", str(csrc), f"-j{int(jobs)}", f"PYTHON={sys.executable}"]
+            r = subprocess.run(make + ["lib"], capture_output=True, text=True)
             if r.returncode != 0 or not os.path.exists(lib):
                 raise RuntimeError(f"building {lib} failed:\n{r.stdout[-4000:]}\n"
                                    f"{r.stderr[-4000:]}")
+            subprocess.run(make + ["native"], capture_output=True, text=True)  # optional
     return lib
 
 
