@@ -131,12 +131,16 @@ int prefill(PyObject *const *x) {
   void *stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
   const size_t need = workspace_bytes(static_cast<int>(T), static_cast<int>(N), static_cast<int>(hqk),
                                       static_cast<int>(hv));
-  PyObject *held = nullptr, *ws = x[12];
+  struct Held {  // given back on every way out, a C++ exception included
+    PyObject *o = nullptr;
+    ~Held() { Py_XDECREF(o); }
+  } held;
+  PyObject *ws = x[12];
   if (ws == Py_None) {
-    ws = held = PyObject_CallFunction(x[13], "iKn", static_cast<int>(dev.index()),
-                                      reinterpret_cast<unsigned long long>(stream),
-                                      static_cast<Py_ssize_t>(need));
-    if (held == nullptr) return 2;
+    ws = held.o = PyObject_CallFunction(x[13], "iKn", static_cast<int>(dev.index()),
+                                        reinterpret_cast<unsigned long long>(stream),
+                                        static_cast<Py_ssize_t>(need));
+    if (ws == nullptr) return 2;
   }
   const at::Tensor *w = plain(ws);
   int rc = 1;
@@ -155,7 +159,6 @@ int prefill(PyObject *const *x) {
                        static_cast<int>(T), scale, po, pn, pw, bytes, stream);
     Py_END_ALLOW_THREADS
   }
-  Py_XDECREF(held);
   return rc;
 }
 

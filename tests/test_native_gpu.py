@@ -1,6 +1,8 @@
 """The native entry of ordinary calls (csrc/gdn_torch.cpp): the same bits as
 the Python path, which takes every other call, errors included."""
 
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -98,3 +100,21 @@ def test_other_calls_take_the_python_path(cuda_device):
     with pytest.raises(ValueError, match="overlaps"):
         decode.kernel(d["q"], d["k"], d["v"], d["state"], d["A_log"], d["a"], d["dt_bias"], d["b"], 0.5,
                       d["v"], torch.empty_like(d["state"]))
+
+
+def test_cached_workspace_is_given_back(cuda_device):
+    # a workspace without an address of its own (vmapped): the call is left to
+    # the Python path, and the tensor is not held
+    d = _dev(O.make_prefill_inputs([100], seed=9), cuda_device)
+    o = torch.empty((100, 8, 128), dtype=torch.bfloat16, device=cuda_device)
+    s = torch.empty((1, 8, 128, 128), device=cuda_device)
+
+    def call(w):
+        held = sys.getrefcount(w)
+        rc = _lib.native().prefill(d["q"], d["k"], d["v"], d["state"], d["A_log"], d["a"], d["dt_bias"],
+                                   d["b"], d["cu_seqlens"], None, o, s, None, lambda *_: w)
+        assert rc == 1
+        assert sys.getrefcount(w) == held
+        return w
+
+    torch.vmap(call)(torch.empty((2, prefill.workspace_bytes(100, 1)), dtype=torch.uint8, device=cuda_device))
