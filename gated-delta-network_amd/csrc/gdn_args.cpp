@@ -287,6 +287,10 @@ int plan_prefill(int T, int N, const Heads &H, const PrefillLayout &L, int varia
   const long long state_units = static_cast<long long>(split ? 3 : N) * H.v * (kDV / 16);
   if (state_units > 0x7fffffffLL) return fail(GDN_ERR_INVALID, "%s: too many sequences", what);
   P.state_grid = cap(state_units, kStatePerCu);
+  if (P.scan) {
+    P.scan_grid = static_cast<long long>(N) * H.v * 4;
+    if (P.scan_more == 0) P.scan_grid = cap(P.scan_grid, kScanPerCu);
+  }
   P.split_grid = split ? static_cast<long long>(L.nt_max - P.split_nt0) * H.v : 0;
   P.early_grid = split && H.v == 8 && state_units + kEarlyGrid <= kNumCus &&
                          P.split_nt0 >= 2 * kEarlyTail

@@ -131,6 +131,15 @@ constexpr int kIntraSplitPerCu = 2;
 // XCD), so that a batch handed to a sequential kernel does not dispatch a
 // full grid (N x 64 workgroups) of idle ones.
 constexpr int kStatePerCu = 2;
+// The same for the fused scan's first segments, of which a batch has N * H.v * 4
+// workgroups: two are resident per CU (their LDS), but the cap lies where an
+// idle grid costs what the launch itself does.  A capped grid deals its units
+// out in a fixed order, which costs batches that do take the chunks more than
+// it saves the others (us per call, uncapped / cap of 2 / 16 / 32 per CU: idle,
+// 4096 x 1 token 896 / 848 / 853 / 850, 512 x 10 157 / 151 / 153 / 154; chunks,
+// 512 sequences of 1..600 tokens 783 / 841 / 795 / 783, 1000 of them 1526 /
+// 1690 / 1575 / 1539).  Cut batches (at most 64 sequences) are not capped.
+constexpr int kScanPerCu = 32;
 
 // What a prefill call launches, decided from (T, N), the head layout and the
 // tuning arguments alone (cu_seqlens is never read on the host).
@@ -147,6 +156,10 @@ struct PrefillPlan {
                     // sequential kernels are the more precise ones, so no batch
                     // leaves them for the scan's sake
   int scan_more;    // most segments beyond the sequences' first ones (0: none is cut)
+  long long scan_grid;  // fused scan: workgroups of the first segments' output; fewer
+                    // than the N * H.v * 4 units they loop over when the device makes
+                    // the path choice (a batch handed to a sequential kernel then does
+                    // not dispatch a grid that grows with N to return at once)
   int split_nt0;    // two-segment scan: first chunk of the second segment; 0 none
   bool intra_split; // WY intra kernel as two workgroups per (chunk, v-head)
   bool loop;        // the state kernel loops over its units in a capped grid

@@ -234,7 +234,8 @@ struct ScanArgs {
   const char *rec;
   char *seg;           // segment maps (SegSlot)
   const int *seg_len;  // chunks of a segment, 0 if the sequences are not cut (nullptr: 0)
-  int out_units;       // first launch: workgroups of the first segments
+  int out_units;       // first launch: units of the first segments' output
+  int out_grid;        // and the workgroups that take them (fewer: each loops)
   Heads H;
   float scale;
 };
@@ -892,24 +893,16 @@ __device__ __forceinline__ void out_unit(const ScanArgs &A, char *smem, const Se
   }
 }
 
-// Launch 1 (SECOND = false): the first segment of every (sequence, v-head)
-// with its output, and the maps of the middle segments.  Launch 2: the other
-// segments with their output.
+// Unit `id` of a launch of scan_chain_kernel: a segment's output or, `map`, a
+// share of a middle segment's map.
 template <bool SECOND>
-__global__ __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void scan_chain_kernel(ScanArgs A) {
-  __shared__ __align__(16) char smem[kScanLds];
+__device__ __forceinline__ void chain_unit(const ScanArgs &A, char *smem, int id, bool map, int seg_len) {
   const Heads &H = A.H;
-  const CoveredRows rows = covered_rows(A.cu, A.cu64, A.N, A.T);
-  if (A.offsets != nullptr && __builtin_amdgcn_readfirstlane(A.offsets[A.N + 1]))
-    return;  // the sequential kernel owns the batch
-  const bool map = !SECOND && static_cast<int>(blockIdx.x) >= A.out_units;
-  const int id = map ? blockIdx.x - A.out_units : blockIdx.x;
   // the same four workgroups for each slot: the quarters of the columns, or the
   // two halves of the offset (0, 1) and of the linear part (2, 3) of a map
   const int h = id % H.v, part = (id / H.v) & 3;
   const int hq = h / H.ratio;
   int s = id / H.v >> 2, seg = 0;
-  const int seg_len = A.seg_len != nullptr ? __builtin_amdgcn_readfirstlane(*A.seg_len) : 0;
   if (SECOND || map) {
     if (seg_len == 0) return;
     // slot number -> (sequence, segment): nseg - 1 segments each here, nseg - 2
@@ -963,7 +956,31 @@ __global__ __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(2,
     map_unit(A, smem, sg, SegSlot{slot0.base + static_cast<size_t>(first) * step, step}, h, hq, part & 1, part >> 1);
   else
     out_unit(A, smem, sg, seg, seg_len, last, slot0, (static_cast<size_t>(s) * H.v + h) * kDV * kDK, h, hq, part);
-  if (!SECOND && !map) zero_rows_outside(A.out, rows, A.T, H.v, blockIdx.x, A.out_units);
+}
+
+// Launch 1 (SECOND = false): the first segment of every (sequence, v-head)
+// with its output, and the maps of the middle segments.  Launch 2: the other
+// segments with their output.  LOOP (launch 1 without maps, which would spill):
+// the output units by a capped grid (PrefillPlan::scan_grid), a workgroup taking
+// every out_grid-th one.
+template <bool SECOND, bool LOOP>
+__global__ __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void scan_chain_kernel(ScanArgs A) {
+  __shared__ __align__(16) char smem[kScanLds];
+  const Heads &H = A.H;
+  const CoveredRows rows = covered_rows(A.cu, A.cu64, A.N, A.T);
+  if (A.offsets != nullptr && __builtin_amdgcn_readfirstlane(A.offsets[A.N + 1]))
+    return;  // the sequential kernel owns the batch
+  const bool map = !SECOND && !LOOP && static_cast<int>(blockIdx.x) >= A.out_grid;
+  int id = map ? blockIdx.x - A.out_grid : blockIdx.x;
+  const int seg_len = A.seg_len != nullptr ? __builtin_amdgcn_readfirstlane(*A.seg_len) : 0;
+  for (;;) {
+    chain_unit<SECOND>(A, smem, id, map, seg_len);
+    if (!LOOP) break;
+    id += A.out_grid;
+    if (id >= A.out_units) break;
+    __syncthreads();  // the unit's LDS is free
+  }
+  if (!SECOND && !map) zero_rows_outside(A.out, rows, A.T, H.v, blockIdx.x, A.out_grid);
 }
 
 int scan_launch(const uint16_t *q, const uint16_t *k, const uint16_t *v, const float *state,
@@ -992,13 +1009,14 @@ int scan_launch(const uint16_t *q, const uint16_t *k, const uint16_t *v, const f
   const ScanArgs A{q, k, v, state, new_state, out, cu, cu64, N, T,
                    P.single ? nullptr : offsets, rec, ws + L.ht,
                    P.scan_more > 0 ? offsets + N + 2 : nullptr,
-                   static_cast<int>(out_units), H, scale};
+                   static_cast<int>(out_units), static_cast<int>(P.scan_grid), H, scale};
   const long long maps = P.scan_more > 1 ? static_cast<long long>(P.scan_more - 1) * H.v * 4 : 0;
-  hipLaunchKernelGGL(scan_chain_kernel<false>, dim3(static_cast<unsigned>(out_units + maps)),
-                     dim3(kScanThreads), 0, stream, A);
+  const auto first = P.scan_grid < out_units ? scan_chain_kernel<false, true> : scan_chain_kernel<false, false>;
+  hipLaunchKernelGGL(first, dim3(static_cast<unsigned>(P.scan_grid + maps)), dim3(kScanThreads), 0,
+                     stream, A);
   if (int rc = check_launch(what)) return rc;
   if (P.scan_more > 0) {
-    hipLaunchKernelGGL(scan_chain_kernel<true>,
+    hipLaunchKernelGGL((scan_chain_kernel<true, false>),
                        dim3(static_cast<unsigned>(static_cast<long long>(P.scan_more) * H.v * 4)),
                        dim3(kScanThreads), 0, stream, A);
     return check_launch(what);

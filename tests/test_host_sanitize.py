@@ -217,3 +217,36 @@ def test_plan_sweep(driver):
             # batches of 2..256 sequences and at most 2560 intra workgroups
             # index themselves in the intra kernel
             assert p["self_index"] == (1 < c[1] <= 256 and 0 < p["intra"] <= 2560), c
+
+
+def _plan(driver, *case):
+    names = ("rc sequential seq_variant choose single form nt0 intra state split out intra_split loop "
+             "self_index early scan more scan_grid").split()
+    return dict(zip(names, map(int, driver(["plan " + " ".join(map(str, case))])[0].split())))
+
+
+@pytest.mark.parametrize("N, tokens, hqk, hv", [(256, 1, 4, 8), (1024, 10, 4, 8), (4096, 10, 4, 8),
+                                                (1 << 20, 4, 4, 8), (512, 24, 16, 32)])
+def test_idle_scan_grid_is_bounded(driver, N, tokens, hqk, hv):
+    # device-chosen batches: the chunks' launches return at once when the
+    # sequential kernel takes the batch, so their grid must not grow with it
+    p = _plan(driver, N * tokens, N, hqk, hv, -1, -1, -1)
+    assert p["choose"] != 0 and p["scan"] == 1
+    assert p["scan_grid"] == min(N * hv * 4, 32 * 256)
+
+
+def test_scan_grid_has_a_workgroup_per_unit_otherwise(driver):
+    # the host's choice, or a batch that may be cut
+    for T, N, hqk, hv in [(8192, 1, 4, 8), (8192, 4, 4, 8), (18000, 300, 4, 8), (126000, 2100, 1, 1),
+                          (4250, 6, 4, 8), (16384, 64, 4, 8)]:
+        p = _plan(driver, T, N, hqk, hv, -1, -1, -1)
+        assert p["scan"] == 1 and (p["choose"] == 0 or p["more"] > 0)
+        assert p["scan_grid"] == N * hv * 4, (T, N)
+
+
+def test_batches_of_the_looped_scan_loop(driver):
+    # the batches of tests/test_scan_gpu.py that are to run the capped grid
+    from test_scan_gpu import LOOPED
+    for lens, (hqk, hv), extra in LOOPED.values():
+        p = _plan(driver, sum(lens) + extra, len(lens), hqk, hv, -1, -1, -1)
+        assert p["scan"] == 1 and p["choose"] != 0 and p["scan_grid"] < len(lens) * hv * 4

@@ -38,7 +38,14 @@ BATCHES = {
 }
 
 
-def _run(inp, dev, heads=(4, 8), in_place=False):
+def _words(ws, T, N):
+    """(chunks, path flag, segment length or operand form) that a batch of N > 1
+    sequences left in its workspace, after the offsets of its sequences."""
+    at = (O.max_chunks(T, N) * 16 + 255) // 256 * 256 + N * 4
+    return ws[at:at + 12].cpu().numpy().view(np.int32).tolist()
+
+
+def _run(inp, dev, heads=(4, 8), in_place=False, workspace=None):
     d = {n: torch.from_numpy(np.ascontiguousarray(inp[n])).to(dev).to(torch.bfloat16)
          for n in ("q", "k", "v", "a", "b")}
     for n in ("A_log", "dt_bias", "cu_seqlens"):
@@ -48,7 +55,7 @@ def _run(inp, dev, heads=(4, 8), in_place=False):
     out = torch.full((T, heads[1], 128), 7.0, dtype=torch.bfloat16, device=dev)
     ns = d["state"] if in_place else torch.full((N, heads[1], 128, 128), 7.0, device=dev)
     prefill.kernel(d["q"], d["k"], d["v"], d["state"], d["A_log"], d["a"], d["dt_bias"], d["b"],
-                   d["cu_seqlens"], inp["scale"], out, ns)
+                   d["cu_seqlens"], inp["scale"], out, ns, workspace=workspace)
     torch.cuda.synchronize()
     return out.float().cpu().numpy(), ns.cpu().numpy()
 
@@ -89,6 +96,31 @@ def test_scan_cut_partial_batch(cuda_device, T, cu):
     o_ref, s_ref = O.prefill_seq_c(**inp)
     o, s = _run(inp, cuda_device)
     assert not o[:cu[0]].any() and not o[cu[-1]:].any()
+    assert_output_close(o, o_ref)
+    assert_state_close(s, s_ref)
+
+
+# Batches whose path the device picks (the chunks, here) in more units than the
+# capped grid has workgroups: (lengths, heads, tokens beyond the sequences).
+LOOPED = {
+    "300": ([200, 0, 500, 37, 1, 129] * 50, (4, 8), 0),
+    "2100": ([3, 40, 0, 17, 130] * 420, (1, 1), 77),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(LOOPED))
+def test_scan_looped_grid(cuda_device, name):
+    lens, heads, extra = LOOPED[name]
+    T, N = sum(lens) + extra, len(lens)
+    print(f"scan looped N={N} T={T} heads={heads}", flush=True)
+    inp = O.make_prefill_inputs(lens[:-1] + [lens[-1] + extra], seed=351, heads=heads)
+    inp["cu_seqlens"][-1] -= extra  # the last rows belong to no sequence: zeros
+    o_ref, s_ref = O.prefill_seq_c(**inp)
+    ws = prefill.alloc_workspace(T, N, cuda_device, heads)
+    o, s = _run(inp, cuda_device, heads, workspace=ws)
+    assert _words(ws, T, N)[1] == 0  # the chunks, not the sequential kernel
+    assert not o[T - extra:].any()
     assert_output_close(o, o_ref)
     assert_state_close(s, s_ref)
 
