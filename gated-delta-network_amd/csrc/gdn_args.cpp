@@ -93,6 +93,15 @@ int plan_multi(const void *q, const void *k, const void *v, int batch, int token
   return GDN_OK;
 }
 
+int rec_tiling(long long groups, long long tokens, bool equal) {
+  if (groups <= 32) return 0;     // 4 rows, 1 wave
+  if (groups <= 64) return 3;     // 8 rows, 1 wave
+  if (groups <= (tokens >= 3 ? 416 : tokens == 2 ? 352 : 256)) return 6;  // 16 rows, 1 wave
+  if (equal && groups > 768 && groups <= 1024 && tokens >= 2 && tokens <= 4) return 9;  // 64 rows, 1 wave
+  if (groups <= 1024) return 8;   // 32 rows, 1 wave
+  return 6;                       // 16 rows, 1 wave
+}
+
 long long max_chunks(long long T, long long N) {
   if (T <= 0 || N <= 0) return 0;
   const long long bound = (T + N * (kChunk - 1)) / kChunk;

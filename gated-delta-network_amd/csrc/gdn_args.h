@@ -60,6 +60,31 @@ constexpr int kDecodeStep = -2;
 int plan_multi(const void *q, const void *k, const void *v, int batch, int tokens, const Heads &H,
                int variant, const char *what, int *kernel);
 
+// Row tiling of the token-by-token kernel (gdn_recurrent.hip) for `groups`
+// (sequence, v-head) pairs of `tokens` tokens: each (`equal`, the rows of a
+// decode batch) or on average (a packed prefill batch, whose longest sequence
+// the host does not know).  From sweeps on MI355X (every tiling, B = 1..512
+// rows of T = 2..6 tokens with 8 v-heads, graph replay over rotating states):
+// few groups -> the smallest row blocks (the serial token loop is spread over
+// the most waves); more -> one wave streaming 8..64 rows.
+// A wave's time grows with its rows times the tokens, so the smaller rows win
+// until a launch of them no longer fits the chip at once: the times jump there,
+// and the next larger block takes over.
+// us per step, 16 / 32 rows: B=40 (320 groups) T=2 9.8 / 10.7, T=4 11.9 / 14.1;
+// B=44 T=2 10.7 / 11.0; B=48 11.8 / 11.2, T=3 11.6 / 13.2; B=52 (416) T=3
+// 13.0 / 13.4, T=4 14.0 / 15.0; B=56 T=3 14.1 / 13.5, T=4 15.0 / 15.1.  32 / 64
+// rows: B=96 (768) T=2 18.4 / 19.8, T=4 21.1 / 25.2; B=104 T=2 22.7 /
+// 20.7, T=4 25.6 / 25.4; B=128 25.5 / 22.8, 29.2 / 28.2, T=5 31.2 / 32.4; B=136
+// T=2 26.8 / 27.9 (B=132).
+// One sequence longer than the rest makes a wave of 64 rows the launch's time,
+// so only equal ones take it (97 prompts of 1..8 tokens 29.0 / 33.3, 96 steps
+// beside one prompt of 192 tokens 216 / 343); for the same reason 16 rows serve
+// uneven batches at least as well as equal ones (50 prompts of 1..8 tokens
+// 17.0 / 18.7, 48 steps beside one of 96 64.9 / 108).
+// One-token sequences (prefill only; decode has its own kernel) are outside
+// that sweep and keep the lines of an earlier one.
+int rec_tiling(long long groups, long long tokens, bool equal);
+
 // Prefill workspace: every region starts on a 256-byte boundary.
 struct PrefillLayout {
   int nt_max;  // upper bound on the chunk count from (T, N) alone

@@ -280,30 +280,6 @@ void launch_rec(long long groups, hipStream_t stream, const uint16_t *q, const u
 int recurrent_num_variants() { return kNumRecVariants + 1; }
 int recurrent_block_variant() { return kNumRecVariants; }
 
-// Built-in tiling from sweeps on MI355X (every tiling, B = 1..512 rows of
-// T = 2..6 tokens with 8 v-heads, graph replay over rotating states): few
-// (sequence, head) groups -> the smallest row blocks (the serial token loop is
-// spread over the most waves); more -> one wave streaming 8..64 rows.
-// A wave's time grows with its rows times the tokens, so the smaller rows win
-// until a launch of them no longer fits the chip at once: the times jump there,
-// and the next larger block takes over.
-// us per step, 16 / 32 rows: B=40 (320 groups) T=2 9.3 / 10.2, T=4 11.5 / 13.9;
-// B=44 T=2 10.3 / 10.5; B=48 11.1 / 10.7, T=3 11.0 / 12.7; B=52 (416) T=3
-// 12.3 / 13.3, T=4 14.0 / 14.9; B=56 T=4 15.3 / 15.2.  32 / 64 rows: B=96 (768)
-// T=2 17.9 / 18.8, T=4 20.1 / 24.3; B=104 21.3 / 19.7, 24.4 / 24.6; B=128
-// 24.0 / 20.8, 27.7 / 26.6, T=5 29.7 / 30.5; B=136 26.6 / 27.5.
-// `tokens`: mean tokens of a sequence.  One-token sequences (prefill only;
-// decode has its own kernel) are outside that sweep and keep the lines of an
-// earlier one.
-int recurrent_default_variant(long long groups, long long tokens) {
-  if (groups <= 32) return 0;     // 4 rows, 1 wave
-  if (groups <= 64) return 3;     // 8 rows, 1 wave
-  if (groups <= (tokens >= 3 ? 416 : tokens == 2 ? 352 : 256)) return 6;  // 16 rows, 1 wave
-  if (groups > 768 && groups <= 1024 && tokens >= 2 && tokens <= 4) return 9;  // 64 rows, 1 wave
-  if (groups <= 1024) return 8;   // 32 rows, 1 wave
-  return 6;                       // 16 rows, 1 wave
-}
-
 int recurrent_launch(const uint16_t *q, const uint16_t *k, const uint16_t *v, const float *state,
                      const float *A_log, const uint16_t *a, const float *dt_bias,
                      const uint16_t *b, const void *cu, int cu64, int num_seqs, int T,
@@ -311,7 +287,7 @@ int recurrent_launch(const uint16_t *q, const uint16_t *k, const uint16_t *v, co
                      float scale, uint16_t *out, float *new_state, hipStream_t stream,
                      int variant, const char *what) {
   const long long groups = static_cast<long long>(num_seqs) * H.v;
-  if (variant < 0) variant = recurrent_default_variant(groups, num_seqs > 0 ? T / num_seqs : 0);
+  if (variant < 0) variant = rec_tiling(groups, num_seqs > 0 ? T / num_seqs : 0, cu == nullptr);
   if (variant == kNumRecVariants)
     return block_launch(q, k, v, state, A_log, a, dt_bias, b, cu, cu64, num_seqs, T, fixed_len,
                         enable, status, H, scale, out, new_state, stream, what);

@@ -11,10 +11,12 @@
 //           variant rec_max rec_variant hqk hv
 //   layout  T N hqk hv
 //   plan    T N hqk hv variant rec_max rec_variant
+//   rec     groups tokens equal
 //
 // decode / multi / prefill print "rc<TAB>message" (the library's status and
 // gdn_last_error text; multi adds the chosen kernel); layout prints
-// "rc nt_max total"; plan prints "rc" and the PrefillPlan fields.
+// "rc nt_max total"; plan prints "rc" and the PrefillPlan fields; rec prints
+// the built-in row tiling.
 #include <stdio.h>
 #include <string.h>
 
@@ -133,6 +135,14 @@ int main() {
         rc = plan_prefill(T, N, H, L, variant, rec_max, rec_variant, kNumRecTilings, "plan", P);
       }
       print_plan(rc, P);
+    } else if (!strcmp(cmd, "rec")) {
+      long long groups, tokens;
+      int equal;
+      if (sscanf(rest, "%lld %lld %d", &groups, &tokens, &equal) != 3) {
+        printf("parse error\n");
+        return 2;
+      }
+      printf("%d\n", rec_tiling(groups, tokens, equal != 0));
     } else {
       printf("unknown command %s\n", cmd);
       return 2;

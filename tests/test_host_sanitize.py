@@ -250,3 +250,18 @@ def test_batches_of_the_looped_scan_loop(driver):
     for lens, (hqk, hv), extra in LOOPED.values():
         p = _plan(driver, sum(lens) + extra, len(lens), hqk, hv, -1, -1, -1)
         assert p["scan"] == 1 and p["choose"] != 0 and p["scan_grid"] < len(lens) * hv * 4
+
+
+def _rec(driver, cases):
+    """Built-in row tiling per (groups, tokens, equal)."""
+    return [int(line) for line in driver([f"rec {g} {t} {int(e)}" for g, t, e in cases])]
+
+
+def test_row_tilings_of_uneven_batches(driver):
+    # a packed batch's mean says nothing of its longest sequence, which a wave of
+    # 64 rows would make the launch's time: it takes at most 32 rows
+    cases = [(g, t, False) for g in range(1, 1400, 7) for t in (1, 2, 3, 4, 5, 9, 100)]
+    for (groups, tokens, _), tiling in zip(cases, _rec(driver, cases)):
+        assert tiling in (0, 3, 6, 8), (groups, tokens)
+        if groups > 416:
+            assert tiling == (8 if groups <= 1024 else 6)
