@@ -97,9 +97,15 @@ int rec_tiling(long long groups, long long tokens, bool equal) {
   if (groups <= 32) return 0;     // 4 rows, 1 wave
   if (groups <= 64) return 3;     // 8 rows, 1 wave
   if (groups <= (tokens >= 3 ? 416 : tokens == 2 ? 352 : 256)) return 6;  // 16 rows, 1 wave
-  if (equal && groups > 768 && groups <= 1024 && tokens >= 2 && tokens <= 4) return 9;  // 64 rows, 1 wave
+  if (equal && groups <= 1024 && tokens >= 2 && tokens <= 4 && groups > (tokens == 4 ? 832 : 768))
+    return 9;                     // 64 rows, 1 wave
   if (groups <= 1024) return 8;   // 32 rows, 1 wave
   return 6;                       // 16 rows, 1 wave
+}
+
+bool rec_packed(int variant, long long groups, long long tokens, bool equal) {
+  if (!equal || tokens < 2 || tokens > 4) return false;
+  return variant == 9 ? groups > 768 : variant == 8 && groups > 416 && groups <= 512;
 }
 
 long long max_chunks(long long T, long long N) {

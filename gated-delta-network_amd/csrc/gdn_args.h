@@ -73,7 +73,7 @@ int plan_multi(const void *q, const void *k, const void *v, int batch, int token
 // us per step, 16 / 32 rows: B=40 (320 groups) T=2 9.8 / 10.7, T=4 11.9 / 14.1;
 // B=44 T=2 10.7 / 11.0; B=48 11.8 / 11.2, T=3 11.6 / 13.2; B=52 (416) T=3
 // 13.0 / 13.4, T=4 14.0 / 15.0; B=56 T=3 14.1 / 13.5, T=4 15.0 / 15.1.  32 / 64
-// rows: B=96 (768) T=2 18.4 / 19.8, T=4 21.1 / 25.2; B=104 T=2 22.7 /
+// rows (packed): B=96 (768) T=2 18.4 / 19.8, T=4 21.1 / 25.2; B=104 T=2 22.7 /
 // 20.7, T=4 25.6 / 25.4; B=128 25.5 / 22.8, 29.2 / 28.2, T=5 31.2 / 32.4; B=136
 // T=2 26.8 / 27.9 (B=132).
 // One sequence longer than the rest makes a wave of 64 rows the launch's time,
@@ -84,6 +84,9 @@ int plan_multi(const void *q, const void *k, const void *v, int batch, int token
 // One-token sequences (prefill only; decode has its own kernel) are outside
 // that sweep and keep the lines of an earlier one.
 int rec_tiling(long long groups, long long tokens, bool equal);
+// Whether that tiling takes its packed form (gdn_recurrent.hip): 32 rows on two
+// waves a SIMD, 64 rows, from two to four tokens each.
+bool rec_packed(int variant, long long groups, long long tokens, bool equal);
 
 // Prefill workspace: every region starts on a 256-byte boundary.
 struct PrefillLayout {

@@ -27,28 +27,31 @@
 //
 // What bounds it: the state's one read and one write when the rows are short
 // (B=64 T=4: 70 MB), and then what a token's step issues beside them.
-// From eight passes on (kPacked) v and o take one memory instruction a token,
-// lane j of a row group carrying the row of pass j mod PASSES, instead of one
-// a pass: a token's memory instructions fall from 4 + 2 PASSES to 6 (us per
-// step, B=64 T=2 / 3 / 4, 32 rows a wave: 12.2 / 14.4 / 16.1 -> 11.6 / 14.1 /
-// 15.5; B=128, 64 rows: 21.9 / 25.4 / 28.4 -> 20.8 / 23.4 / 26.6).  With four
-// passes it gained nothing (B=64 T=2 13.6 -> 14.3); with eight, a ring of four
-// tokens instead of two lost once two waves a SIMD no longer held the launch
-// (B=128 T=4 27.3 -> 30.2), and registers held to four waves a SIMD cost more
-// (B=64 T=4 15.5 -> 19.1).
+// PACKED: v and o take one memory instruction a token, lane j of a row group
+// carrying the row of pass j mod PASSES, instead of one a pass: a token's memory
+// instructions fall from 4 + 2 PASSES to 6, for a broadcast and a select a pass.
+// It pays where the memory instructions are what a short row waits for, and
+// costs elsewhere (us per step of B rows of T tokens, plain / packed; 32
+// rows a wave, B=64 T=2 / 3 / 4: 12.8 / 12.3, 14.6 / 14.3, 16.3 / 15.9, B=96:
+// 18.4 / 18.9, 18.4 / 19.0, 21.1 / 21.1, B=112 T=5 28.5 / 30.3; 64 rows, B=128:
+// 24.1 / 22.8, 27.0 / 25.2, 30.3 / 28.2; prompts of one token, 32 rows, 66 of
+// them 13.4 / 14.9): rec_packed has the lines.  With four passes it gained
+// nothing (B=64 T=2 13.6 -> 14.3); with eight, a ring of four tokens instead of
+// two lost once two waves a SIMD no longer held the launch (B=128 T=4 27.3 ->
+// 30.2), and registers held to four waves a SIMD cost more (B=64 T=4 15.5 ->
+// 19.1).
 #include "gdn_device.h"
 #include "gdn_host.h"
 
 namespace gdn {
 
-template <int PASSES>
+template <int PASSES, bool PACKED>
 struct TokenIn {
-  static constexpr bool kPacked = PASSES >= 8;
   u16x4 k0, k1, q0, q1;
-  uint16_t v[kPacked ? 1 : PASSES];
+  uint16_t v[PACKED ? 1 : PASSES];
 };
 
-template <int WAVES, int PASSES>
+template <int WAVES, int PASSES, bool PACKED>
 __global__ __launch_bounds__(64 * WAVES) void recurrent_kernel(
     const uint16_t *__restrict__ q, const uint16_t *__restrict__ k,
     const uint16_t *__restrict__ v, const float *state, const float *__restrict__ A_log,
@@ -117,7 +120,7 @@ __global__ __launch_bounds__(64 * WAVES) void recurrent_kernel(
   if (len > 0) {
     const float rate = expf(A_log[h]);
     const float dtb = dt_bias[h];
-    auto load_token = [&](int t, TokenIn<PASSES> &x) {
+    auto load_token = [&](int t, TokenIn<PASSES, PACKED> &x) {
       const size_t tok = static_cast<size_t>(bos) + t;
       const uint16_t *kp = k + (tok * H.qk + hq) * kDK + c4;
       const uint16_t *qp = q + (tok * H.qk + hq) * kDK + c4;
@@ -126,7 +129,7 @@ __global__ __launch_bounds__(64 * WAVES) void recurrent_kernel(
       x.q0 = *reinterpret_cast<const u16x4 *>(qp);
       x.q1 = *reinterpret_cast<const u16x4 *>(qp + 64);
       const uint16_t *vp = v + (tok * H.v + h) * kDV + row0;
-      if constexpr (TokenIn<PASSES>::kPacked) {
+      if constexpr (PACKED) {
         x.v[0] = vp[4 * jl];
       } else {
 #pragma unroll
@@ -137,7 +140,7 @@ __global__ __launch_bounds__(64 * WAVES) void recurrent_kernel(
     // One token: x holds its k, q, v; (g, beta) its gating.  Every lane of a
     // row group holds the row's o, so all 16 store the same two bytes, or
     // those of pass jl (one coalesced write), and no lane needs a branch.
-    auto step = [&](const TokenIn<PASSES> &x, int t, float g, float beta) {
+    auto step = [&](const TokenIn<PASSES, PACKED> &x, int t, float g, float beta) {
       float kf[8], qf[8];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -151,7 +154,7 @@ __global__ __launch_bounds__(64 * WAVES) void recurrent_kernel(
       for (int e = 0; e < 8; ++e) pkq = fmaf(kf[e], qf[e], pkq);
       const float kq = row16_sum(pkq);
       float vl = 0.f, ov = 0.f;  // this lane's pass jl of v and o
-      if constexpr (TokenIn<PASSES>::kPacked) vl = bf16_to_f32(x.v[0]);
+      if constexpr (PACKED) vl = bf16_to_f32(x.v[0]);
       uint16_t *op = out + ((static_cast<size_t>(bos) + t) * H.v + h) * kDV + row0;
 #pragma unroll
       for (int p = 0; p < PASSES; ++p) {
@@ -166,7 +169,7 @@ __global__ __launch_bounds__(64 * WAVES) void recurrent_kernel(
         const float sk = row16_sum(sk0 + sk1);
         const float sq = row16_sum(sq0 + sq1);
         float vp;
-        if constexpr (TokenIn<PASSES>::kPacked)
+        if constexpr (PACKED)
           vp = row_bcast16(vl, p);
         else
           vp = bf16_to_f32(x.v[p]);
@@ -177,12 +180,12 @@ __global__ __launch_bounds__(64 * WAVES) void recurrent_kernel(
           Sa[p][e] = fmaf(vn, kf[e], g * Sa[p][e]);
           Sb[p][e] = fmaf(vn, kf[4 + e], g * Sb[p][e]);
         }
-        if constexpr (TokenIn<PASSES>::kPacked)
+        if constexpr (PACKED)
           ov = jl == p ? o : ov;
         else
           op[4 * p] = f32_to_bf16(o);
       }
-      if constexpr (TokenIn<PASSES>::kPacked) op[4 * jl] = f32_to_bf16(ov);
+      if constexpr (PACKED) op[4 * jl] = f32_to_bf16(ov);
     };
 
     // Everything is loaded ahead of use by unconditional loads (indices past
@@ -199,7 +202,7 @@ __global__ __launch_bounds__(64 * WAVES) void recurrent_kernel(
       return (static_cast<size_t>(bos) + (t < last ? t : last)) * H.v + h;
     };
     uint16_t a_raw = a[gate_idx(0)], b_raw = b[gate_idx(0)];
-    TokenIn<PASSES> ring[kDepth];
+    TokenIn<PASSES, PACKED> ring[kDepth];
 #pragma unroll
     for (int r = 0; r < kDepth; ++r) load_token(r < last ? r : last, ring[r]);
     // Gating of the turn's tokens, token t0 + (lane % kDepth) in each lane.
@@ -261,14 +264,14 @@ constexpr RecVariant kRecVariants[] = {
 constexpr int kNumRecVariants = sizeof(kRecVariants) / sizeof(kRecVariants[0]);
 static_assert(kNumRecVariants == kNumRecTilings, "the tiling count is shared with the host code");
 
-template <int W, int P>
+template <int W, int P, bool PACKED>
 void launch_rec(long long groups, hipStream_t stream, const uint16_t *q, const uint16_t *k,
                 const uint16_t *v, const float *state, const float *A_log, const uint16_t *a,
                 const float *dt_bias, const uint16_t *b, const void *cu, int cu64, int N, int T,
                 int fixed_len, const int *enable, int *status, const Heads &H, float scale,
                 uint16_t *out, float *new_state) {
   const long long blocks = groups * (kDV / (4 * W * P));
-  hipLaunchKernelGGL((recurrent_kernel<W, P>), dim3(static_cast<unsigned>(blocks)), dim3(64 * W),
+  hipLaunchKernelGGL((recurrent_kernel<W, P, PACKED>), dim3(static_cast<unsigned>(blocks)), dim3(64 * W),
                      0, stream, q, k, v, state, A_log, a, dt_bias, b, cu, cu64, N, T, fixed_len,
                      enable, status, H, scale, out, new_state);
 }
@@ -287,7 +290,8 @@ int recurrent_launch(const uint16_t *q, const uint16_t *k, const uint16_t *v, co
                      float scale, uint16_t *out, float *new_state, hipStream_t stream,
                      int variant, const char *what) {
   const long long groups = static_cast<long long>(num_seqs) * H.v;
-  if (variant < 0) variant = rec_tiling(groups, num_seqs > 0 ? T / num_seqs : 0, cu == nullptr);
+  const long long tokens = num_seqs > 0 ? T / num_seqs : 0;
+  if (variant < 0) variant = rec_tiling(groups, tokens, cu == nullptr);
   if (variant == kNumRecVariants)
     return block_launch(q, k, v, state, A_log, a, dt_bias, b, cu, cu64, num_seqs, T, fixed_len,
                         enable, status, H, scale, out, new_state, stream, what);
@@ -296,20 +300,23 @@ int recurrent_launch(const uint16_t *q, const uint16_t *k, const uint16_t *v, co
   const RecVariant rv = kRecVariants[variant];
   if (groups * (kDV / (4 * rv.waves * rv.passes)) > 0x7fffffffLL)
     return fail(GDN_ERR_INVALID, "%s: too many sequences for one launch", what);
-#define GDN_REC(W, P)                                                                          \
-  if (rv.waves == W && rv.passes == P)                                                        \
-    launch_rec<W, P>(groups, stream, q, k, v, state, A_log, a, dt_bias, b, cu, cu64, num_seqs, \
-                     T, fixed_len, enable, status, H, scale, out, new_state);
-  GDN_REC(1, 1)
-  GDN_REC(2, 1)
-  GDN_REC(4, 1)
-  GDN_REC(1, 2)
-  GDN_REC(2, 2)
-  GDN_REC(4, 2)
-  GDN_REC(1, 4)
-  GDN_REC(4, 4)
-  GDN_REC(1, 8)
-  GDN_REC(1, 16)
+  const bool packed = rec_packed(variant, groups, tokens, cu == nullptr);
+#define GDN_REC(W, P, PACKED)                                                                  \
+  if (rv.waves == W && rv.passes == P && packed == PACKED)                                    \
+    launch_rec<W, P, PACKED>(groups, stream, q, k, v, state, A_log, a, dt_bias, b, cu, cu64,   \
+                             num_seqs, T, fixed_len, enable, status, H, scale, out, new_state);
+  GDN_REC(1, 1, false)
+  GDN_REC(2, 1, false)
+  GDN_REC(4, 1, false)
+  GDN_REC(1, 2, false)
+  GDN_REC(2, 2, false)
+  GDN_REC(4, 2, false)
+  GDN_REC(1, 4, false)
+  GDN_REC(4, 4, false)
+  GDN_REC(1, 8, false)
+  GDN_REC(1, 8, true)
+  GDN_REC(1, 16, false)
+  GDN_REC(1, 16, true)
 #undef GDN_REC
   return check_launch(what);
 }

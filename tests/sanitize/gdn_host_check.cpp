@@ -11,12 +11,12 @@
 //           variant rec_max rec_variant hqk hv
 //   layout  T N hqk hv
 //   plan    T N hqk hv variant rec_max rec_variant
-//   rec     groups tokens equal
+//   rec     groups tokens equal variant
 //
 // decode / multi / prefill print "rc<TAB>message" (the library's status and
 // gdn_last_error text; multi adds the chosen kernel); layout prints
 // "rc nt_max total"; plan prints "rc" and the PrefillPlan fields; rec prints
-// the built-in row tiling.
+// the built-in tiling and whether `variant` (-1: that one) is packed.
 #include <stdio.h>
 #include <string.h>
 
@@ -137,12 +137,13 @@ int main() {
       print_plan(rc, P);
     } else if (!strcmp(cmd, "rec")) {
       long long groups, tokens;
-      int equal;
-      if (sscanf(rest, "%lld %lld %d", &groups, &tokens, &equal) != 3) {
+      int equal, variant;
+      if (sscanf(rest, "%lld %lld %d %d", &groups, &tokens, &equal, &variant) != 4) {
         printf("parse error\n");
         return 2;
       }
-      printf("%d\n", rec_tiling(groups, tokens, equal != 0));
+      const int tiling = rec_tiling(groups, tokens, equal != 0);
+      printf("%d %d\n", tiling, rec_packed(variant < 0 ? tiling : variant, groups, tokens, equal != 0) ? 1 : 0);
     } else {
       printf("unknown command %s\n", cmd);
       return 2;

@@ -253,15 +253,25 @@ def test_batches_of_the_looped_scan_loop(driver):
 
 
 def _rec(driver, cases):
-    """Built-in row tiling per (groups, tokens, equal)."""
-    return [int(line) for line in driver([f"rec {g} {t} {int(e)}" for g, t, e in cases])]
+    """(built-in tiling, whether `variant` or it is packed) per (groups, tokens, equal, variant)."""
+    out = driver([f"rec {g} {t} {int(e)} {v}" for g, t, e, v in cases])
+    return [tuple(map(int, line.split())) for line in out]
 
 
 def test_row_tilings_of_uneven_batches(driver):
     # a packed batch's mean says nothing of its longest sequence, which a wave of
     # 64 rows would make the launch's time: it takes at most 32 rows
-    cases = [(g, t, False) for g in range(1, 1400, 7) for t in (1, 2, 3, 4, 5, 9, 100)]
-    for (groups, tokens, _), tiling in zip(cases, _rec(driver, cases)):
-        assert tiling in (0, 3, 6, 8), (groups, tokens)
+    cases = [(g, t, False, -1) for g in range(1, 1400, 7) for t in (1, 2, 3, 4, 5, 9, 100)]
+    for (groups, tokens, _, _), (tiling, packed) in zip(cases, _rec(driver, cases)):
+        assert tiling in (0, 3, 6, 8) and not packed, (groups, tokens)
         if groups > 416:
             assert tiling == (8 if groups <= 1024 else 6)
+
+
+def test_row_tilings_of_equal_rows(driver):
+    want = {(352, 2): (6, 0), (353, 2): (8, 0), (416, 3): (6, 0), (417, 2): (8, 1), (512, 4): (8, 1),
+            (513, 4): (8, 0), (512, 5): (8, 0), (768, 3): (8, 0), (769, 2): (9, 1), (832, 4): (8, 0),
+            (833, 4): (9, 1), (1024, 5): (8, 0), (1024, 3): (9, 1), (1025, 3): (6, 0)}
+    got = _rec(driver, [(g, t, True, -1) for g, t in want])
+    assert dict(zip(want, got)) == want
+    assert _rec(driver, [(600, 3, True, 9)]) == [(8, 0)]  # as asked for, plain

@@ -295,8 +295,8 @@ def test_multi_token_decode_tilings_are_identical(cuda_device):
 
 # Both sides of the lines between 16, 32 and 64 rows a wave (44, 52, 96 and 128
 # rows of 8 v-heads), token counts around the two-token ring of the larger ones.
-@pytest.mark.parametrize("B, T", [(44, 2), (45, 2), (52, 3), (53, 3), (96, 3), (97, 2), (97, 3),
-                                  (128, 4), (128, 5), (129, 2)])
+@pytest.mark.parametrize("B, T", [(44, 2), (45, 2), (52, 3), (53, 3), (64, 4), (65, 2), (96, 3), (97, 2),
+                                  (97, 3), (104, 4), (128, 4), (128, 5), (129, 2)])
 def test_multi_token_decode_tiling_lines(cuda_device, B, T):
     inp, dec = _multi_inputs(B, T, seed=35 + B + T)
     d = _to_dev(dec, cuda_device)
