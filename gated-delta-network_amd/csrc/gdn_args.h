@@ -144,7 +144,8 @@ constexpr int kRecurrentMaxLen = 96;
 // chunks).
 constexpr int kSplitMinChunks = 9;
 
-// Chunks of the shortest sequence that the fused scan may cut.
+// Chunks that the longest sequence could have, by (T, N) alone, from which on a
+// batch gets the second launch of the cut scan (segment_choice decides there).
 constexpr int kScanCutMin = 20;
 
 // Compute units of the target (MI355X: 256).  The WY intra kernel runs each

@@ -59,35 +59,11 @@ __device__ __forceinline__ int wave_sum(int x) {
          __builtin_amdgcn_readlane(x, 32) + __builtin_amdgcn_readlane(x, 48);
 }
 
-// Fused scan: the segment length (chunks) for sequences of n chunks each (lane
-// s of the one wave that calls it: sequence s, at most 64), 0 to leave them
-// whole.  A sequence cut into P segments of len chunks runs two chains of len
-// steps, the middle segments' maps and then the outputs, and up to P - 2 map
-// applications, instead of one chain of P len steps; at most max_more segments
-// beyond the sequences' first ones (the second launch's grid), and as many
-// workgroups in the first.  Times in microseconds, fitted to sweeps on MI355X
-// (N = 1..8 sequences of 512..8192 tokens): a step 1.5 alone on a CU, 1.25 of
-// a CU's time when it holds two; a map's two 64-column halves 1.8.
+// Fused scan: the segment length (segment_choice) for sequences of n chunks
+// each (lane s of the one wave that calls it: sequence s, at most 64).
 __device__ __forceinline__ int segment_length(int n, int max_more, int hv) {
-  const int longest = static_cast<int>(wave_max(static_cast<float>(n)));
-  int len = (longest + 7) / 8;
-  len = len < kMinSegment ? kMinSegment : len;
-  const int m = n > 0 ? n - 1 : 0;
-  int mids = 0;
-  for (;;) {
-    if (len >= longest) return 0;
-    const int more = m / len;  // segments beyond the first
-    mids = wave_sum(more > 1 ? more - 1 : 0);
-    if (wave_sum(more) <= max_more && wave_sum(n >= len ? 1 : 0) + mids <= max_more) break;
-    len += len < 8 ? 1 : len / 8;
-  }
-  const float cus = static_cast<float>(hv * 4) / 256.0f;  // CUs of one slot's workgroups
-  const float work = 1.25f * cus * static_cast<float>(wave_sum(n));
-  const float maps = 1.8f * cus * static_cast<float>(mids * len);
-  const float whole = fmaxf(1.5f * static_cast<float>(longest), work);
-  const float chain = 3.6f * static_cast<float>(len) +
-                      2.0f * static_cast<float>((longest + len - 1) / len - 2) + 6.0f;
-  return fmaxf(chain, work + maps + 12.0f) < whole ? len : 0;
+  return segment_choice(static_cast<int>(wave_max(static_cast<float>(n))), max_more, hv,
+                        [n](auto f) { return wave_sum(f(n)); });
 }
 
 // Chunk c of the table; for a single sequence (one.cu != nullptr) there is no

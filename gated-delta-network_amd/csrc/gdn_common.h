@@ -106,8 +106,69 @@ constexpr float kSeqChoiceMargin = 4.0f;
 constexpr int kSelfIndexMax = 256;
 constexpr long long kSelfIndexMaxGrid = 2560;
 
-// Shortest segment of the fused scan (gdn_scan.hip), in chunks.
+// Shortest segment of the fused scan (gdn_scan.hip), in chunks, and shortest
+// longest sequence of a batch whose sequences it cuts.
 constexpr int kMinSegment = 4;
+constexpr int kMinCut = 16;
+
+// Fused scan: the segment length (chunks) for a batch whose longest sequence has
+// `longest` chunks, 0 to leave the sequences whole.  sum(f) is the sum of f(n)
+// over the sequences, n their chunks (on the device each lane holds one).
+// A sequence cut into P segments of len chunks runs two chains of len steps, the
+// middle segments' maps and then the outputs, and P - 2 map applications,
+// instead of one chain of P len steps; at most max_more segments beyond the
+// sequences' first ones (the second launch's grid), and as many workgroups in
+// the first.
+// Of the lengths that cut the longest sequence into eight to three, from the
+// shortest on, one is taken over a shorter one if its estimate is a tenth
+// lower, and any if it beats the whole sequences.  The shortest that fits the
+// grid is often not the best: as soon as a launch has more workgroups than
+// compute units, its steps take longer, and by more where the v-heads are no
+// multiple of the 8 XCDs (the four workgroups that read one head's operands then
+// run on different ones, each with its own L2).  us, shortest / best: 3 x 20
+// chunks of 8 v-heads, 4 chunks 53.3 / 7 chunks 45.5; 32 chunks of 10 v-heads, 4
+// chunks 53.2 / 5 chunks 46.2; 2 x 32 of 8, 4 chunks 58.3 / 7 chunks 49.4.
+// Estimates in microseconds, fitted to every length of 1450 batches of N = 1..8
+// equal sequences of 16..128 chunks with 1..64 v-heads and 127 uneven ones of
+// 2..64 sequences.
+template <class Sum>
+__host__ __device__ inline int segment_choice(int longest, int max_more, int hv, Sum sum) {
+  if (longest < kMinCut) return 0;
+  const float cus = static_cast<float>(hv) * (4.0f / 256.0f);  // CUs of one slot's workgroups
+  const bool xcds = hv % 8 == 0;
+  // step time relative to a CU of its own, w workgroups a CU
+  auto share = [](float w) { return w <= 1.0f ? 1.0f : 1.15f + 0.4f * (w - 1.0f); };
+  const float work = 1.05f * cus * static_cast<float>(sum([](int n) { return n; }));
+  const float w0 = fminf(cus * static_cast<float>(sum([=](int n) { return 2 * n > longest ? 1 : 0; })), 2.0f);
+  const float whole = fmaxf(1.3f * share(w0) * static_cast<float>(longest) + (w0 > 1.0f ? 4.0f : 0.0f), work);
+  int best_len = 0;
+  float best = 0.0f;
+  for (int parts = 8; parts >= 3; --parts) {
+    int len = (longest + parts - 1) / parts;
+    len = len < kMinSegment ? kMinSegment : len;
+    if (2 * len >= longest) continue;
+    // segments beyond the first, maps, first segments that are full: at most
+    // eight of each a sequence, of at most 64
+    const int counts = sum([=](int n) {
+      const int more = n > len ? (n - 1) / len : 0;
+      return more | (more > 1 ? more - 1 : 0) << 10 | (n >= len ? 1 : 0) << 20;
+    });
+    const int second = counts & 1023, mids = (counts >> 10) & 1023, first = (counts >> 20) + mids;
+    if (first > max_more || second > max_more) continue;
+    const float w = cus * static_cast<float>(first > second ? first : second);
+    const float step = 2.9f * share(w) * (w > 1.0f && !xcds ? 1.5f : 1.0f);
+    const float chain = step * static_cast<float>(len) +
+                        1.5f * static_cast<float>((longest + len - 1) / len - 2) +
+                        (w > 1.0f ? 12.0f : 4.0f) + (xcds ? 0.0f : 3.0f * w);
+    const float est = fmaxf(chain, work + 1.2f * cus * static_cast<float>(mids * len) + 8.0f);
+    if (best_len == 0 || est < 0.9f * best) {
+      best = est;
+      best_len = len;
+    }
+    if (w <= 1.0f) break;  // a longer segment only has fewer workgroups yet
+  }
+  return best_len != 0 && best < whole ? best_len : 0;
+}
 
 // First chunk of the second segment of a two-segment scan over nt chunks.
 __host__ __device__ inline int split_first(int nt) { return (nt + 1) / 2; }

@@ -12,13 +12,17 @@
 //   layout  T N hqk hv
 //   plan    T N hqk hv variant rec_max rec_variant
 //   rec     groups tokens equal variant
+//   seg     hv max_more n n ...
 //
 // decode / multi / prefill print "rc<TAB>message" (the library's status and
 // gdn_last_error text; multi adds the chosen kernel); layout prints
 // "rc nt_max total"; plan prints "rc" and the PrefillPlan fields; rec prints
-// the built-in tiling and whether `variant` (-1: that one) is packed.
+// the built-in tiling and whether `variant` (-1: that one) is packed; seg prints the
+// fused scan's segment length for sequences of n chunks each.
 #include <stdio.h>
 #include <string.h>
+
+#include <vector>
 
 #include "gdn_args.h"
 
@@ -144,6 +148,21 @@ int main() {
       }
       const int tiling = rec_tiling(groups, tokens, equal != 0);
       printf("%d %d\n", tiling, rec_packed(variant < 0 ? tiling : variant, groups, tokens, equal != 0) ? 1 : 0);
+    } else if (!strcmp(cmd, "seg")) {
+      int hv, max_more, used = 0, x;
+      if (sscanf(rest, "%d %d%n", &hv, &max_more, &used) != 2) {
+        printf("parse error\n");
+        return 2;
+      }
+      std::vector<int> chunks;
+      for (const char *at = rest + used; sscanf(at, "%d%n", &x, &used) == 1; at += used) chunks.push_back(x);
+      int longest = 0;
+      for (int c : chunks) longest = c > longest ? c : longest;
+      printf("%d\n", segment_choice(longest, max_more, hv, [&](auto f) {
+               int total = 0;
+               for (int c : chunks) total += f(c);
+               return total;
+             }));
     } else {
       printf("unknown command %s\n", cmd);
       return 2;

@@ -275,3 +275,37 @@ def test_row_tilings_of_equal_rows(driver):
     got = _rec(driver, [(g, t, True, -1) for g, t in want])
     assert dict(zip(want, got)) == want
     assert _rec(driver, [(600, 3, True, 9)]) == [(8, 0)]  # as asked for, plain
+
+
+def _segment_workgroups(chunks, length, hv):
+    """Workgroups of the scan's two launches that work on full segments or maps."""
+    more = [(n - 1) // length if n else 0 for n in chunks]
+    maps = sum(max(m - 1, 0) for m in more)
+    return 4 * hv * (sum(n >= length for n in chunks) + maps), 4 * hv * sum(more)
+
+
+def test_segment_length(driver):
+    # equal sequences: within the grids, and one workgroup a compute unit where a
+    # length allows it that cuts the longest sequence into three or more
+    cases = [(hv, 128 // hv, [c] * n) for hv in (1, 2, 3, 4, 6, 8, 10, 12, 16, 18, 24, 32) for n in (1, 2, 3, 4, 8)
+             for c in (8, 15, 16, 20, 24, 32, 40, 64, 128) if hv * n <= 64]
+    got = driver([f"seg {hv} {m} {' '.join(map(str, n))}" for hv, m, n in cases])
+    cut = 0
+    for (hv, max_more, chunks), length in zip(cases, map(int, got)):
+        if length == 0:
+            continue
+        cut += 1
+        longest = max(chunks)
+        assert longest >= 16 and 4 <= length and 2 * length < longest
+        assert max(_segment_workgroups(chunks, length, hv)) <= 4 * hv * max_more
+        if length > 4:  # no shorter length of one workgroup a unit was left out
+            parts = -(-longest // length) + 1
+            shorter = max(-(-longest // parts), 4)
+            assert parts > 8 or shorter == length or max(_segment_workgroups(chunks, shorter, hv)) > 256
+    assert cut > 150
+    # batches that the shortest length that fits the grid made slower than the
+    # operand forms: 8 v-heads 3 x 20 chunks (4 chunks: 53.3 us, forms 47.0, 7:
+    # 45.5), 10 v-heads 32 and 64 chunks, 16 v-heads 32 chunks, 6 v-heads 3 x 24
+    for hv, chunks, want in [(8, [20] * 3, 7), (10, [32], 5), (10, [64], 10), (16, [32], 7), (6, [24] * 3, 6),
+                             (8, [32] * 2, 7), (8, [128], 16), (8, [15] * 4, 0)]:
+        assert driver([f"seg {hv} {128 // hv} {' '.join(map(str, chunks))}"]) == [str(want)], (hv, chunks)
