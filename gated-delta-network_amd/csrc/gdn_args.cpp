@@ -215,16 +215,27 @@ int check_prefill_args(const gdn_bf16 *q, const gdn_bf16 *k, const gdn_bf16 *v, 
 }
 
 // Whether the chunks go through the fused scan (gdn_scan.hip) or the
-// operand-form pipeline: the scan, except for at most 8 (sequence, v-head)
-// groups of a middling chain, too short to be cut (segment_length) and long
-// enough for the pipeline's shorter step to pay for its third launch (us,
-// operand forms / scan: 1x640 28.2 / 26.6, 1x768 29.4 / 29.7, 1x1024 30.8 /
-// 35.4, 1x2048 39.9 / 40.0, 1x2560 49.0 / 44.5; 2x1024 38.2 / 37.6; with two
-// v-heads 1x4096 47.1 / 50.1, 2x1024 33.8 / 36.6, 2x2048 45.7 / 41.0).
+// operand-form pipeline: the scan, except for few (sequence, v-head) groups of a
+// middling chain, too short to be cut (segment_choice) and long enough for the
+// pipeline's shorter step to pay for its third launch.  Lines from sweeps of
+// both on MI355X (N = 1..8 equal sequences of 4..256 chunks with 1..64 v-heads;
+// us, operand forms / scan):
+//  * one sequence: the pipeline has the two-segment scan (up to 10 v-heads), so
+//    the line falls with the v-heads: 8 of them 11 chunks 28.1 / 26.1, 12 29.4 /
+//    29.7, 16 30.8 / 35.4, 32 39.9 / 40.0, 36 46 / 43; 4 of them 64 chunks 51.4
+//    / 53.5, 80 61 / 59; 10 of them 16 chunks 33.7 / 37.4, 26 43 / 42; one of
+//    them 128 chunks 72.2 / 74.4;
+//  * more sequences, up to 8 groups: 2 x 1024 tokens of two v-heads 33.8 / 36.6,
+//    of four 38.2 / 37.6, 2 x 2048 of two 45.7 / 41.0;
+//  * up to 16 groups of 3, 5, 6 or 7 v-heads (no multiple or divisor of the 8
+//    XCDs): 4 x 16 chunks of three 37.1 / 40.1, 3 x 16 of five 38.8 / 40.8; 4 x
+//    24 of three 48.0 / 47.0.
 static bool scan_wins(int nt, int N, const Heads &H) {
   const long long mean = (static_cast<long long>(nt) + N - 1) / N;
   const long long groups = static_cast<long long>(N) * H.v;
-  return groups > 8 || mean <= 11 || mean >= (groups <= 2 ? 80 : 33);
+  if (N == 1) return H.v >= 16 || nt < (H.v <= 8 ? 12 : H.v <= 11 ? 14 : 16) || groups * nt > 256;
+  if (groups <= 8) return mean <= 11 || mean >= (groups <= 2 ? 80 : 33);
+  return groups > 16 || 8 % H.v == 0 || H.v > 7 || mean <= 13 || mean >= 21;
 }
 
 int plan_prefill(int T, int N, const Heads &H, const PrefillLayout &L, int variant, int rec_max,

@@ -309,3 +309,18 @@ def test_segment_length(driver):
     for hv, chunks, want in [(8, [20] * 3, 7), (10, [32], 5), (10, [64], 10), (16, [32], 7), (6, [24] * 3, 6),
                              (8, [32] * 2, 7), (8, [128], 16), (8, [15] * 4, 0)]:
         assert driver([f"seg {hv} {128 // hv} {' '.join(map(str, chunks))}"]) == [str(want)], (hv, chunks)
+
+
+def test_scan_leaves_short_chains_to_the_operand_forms(driver):
+    # one sequence of nt chunks, by v-heads: the lines between the two
+    for hv, lo, hi in [(1, 12, 256), (2, 12, 128), (4, 12, 64), (8, 12, 32), (10, 14, 25), (12, 16, 21)]:
+        for nt in (1, 11, lo - 1, lo, (lo + hi) // 2, hi, hi + 1, 2 * hi):
+            p = _plan(driver, 64 * nt, 1, 1, hv, -1, -1, -1)
+            assert p["scan"] == (not lo <= nt <= hi), (hv, nt)
+    for hv in (16, 24, 32):
+        assert all(_plan(driver, 64 * nt, 1, 1, hv, -1, -1, -1)["scan"] for nt in (12, 16, 20, 32))
+    # several: up to 8 groups by the mean; more only beside an odd head count
+    for N, hv, mean, scan in [(2, 4, 20, 0), (2, 4, 40, 1), (3, 4, 16, 1), (4, 3, 16, 0), (4, 3, 24, 1),
+                              (2, 8, 16, 1), (3, 6, 16, 1)]:
+        assert _plan(driver, 64 * mean * N - 64 * N, N, 1, hv, -1, -2, -1)["scan"] == 0
+        assert _plan(driver, 64 * mean * N - 64 * N, N, 1, hv, -1, -1, -1)["scan"] == scan, (N, hv, mean)
