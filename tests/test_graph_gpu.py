@@ -236,16 +236,17 @@ def test_prefill_release_workspaces(cuda_device):
     assert_state_close(outs[0][1].cpu().numpy(), s_ref)
 
 
-@pytest.mark.parametrize("T", [2500, 4500])
-def test_prefill_graph_replays_two_segment_scan(cuda_device, T):
-    # One sequence of 2500 tokens (40 chunks: the two-segment scan, its
-    # second-segment output kernel and the new_state tiles), or of 4500 (71
-    # chunks: the state launch also computes the first 21 chunks' output,
-    # with progress words the intra launch zeroes), captured once and
-    # replayed with new inputs; every replay equals the eager call.
+@pytest.mark.parametrize("T, variant", [(2500, -1), (4500, -1), (2500, 3), (4500, 3)])
+def test_prefill_graph_replays_two_segment_scan(cuda_device, T, variant):
+    # One sequence captured once and replayed with new inputs; every replay
+    # equals the eager call.  Built in (-1): the fused scan, cut into segments.
+    # Variant 3: the operand forms' two-segment scan of 2500 tokens (40 chunks:
+    # its second-segment output kernel and the new_state tiles), or of 4500 (71
+    # chunks: the state launch also computes the first 21 chunks' output, with
+    # progress words the intra launch zeroes on every replay).
     dev = cuda_device
     N = 1
-    print(f"prefill graph two-segment T={T}", flush=True)
+    print(f"prefill graph two-segment T={T} variant={variant}", flush=True)
     st = _prefill_static(T, N, dev)
     inp = O.make_prefill_inputs([T], seed=50)
     _fill_prefill(st, inp)
@@ -256,7 +257,8 @@ def test_prefill_graph_replays_two_segment_scan(cuda_device, T):
 
     def call(o, s):
         prefill.kernel(st["q"], st["k"], st["v"], st["state"], st["A_log"], st["a"],
-                       st["dt_bias"], st["b"], st["cu_seqlens"], scale, o, s, workspace=ws)
+                       st["dt_bias"], st["b"], st["cu_seqlens"], scale, o, s, variant=variant,
+                       workspace=ws)
 
     side = torch.cuda.Stream(device=dev)
     side.wait_stream(torch.cuda.current_stream(dev))

@@ -172,8 +172,13 @@ def test_plan_sweep(driver):
         f = [int(x) for x in got.split()]
         plans[c] = dict(rc=f[0], sequential=f[1], seq_variant=f[2], choose=f[3], single=f[4],
                         form=f[5], nt0=f[6], intra=f[7], state=f[8], split=f[9], out=f[10],
-                        intra_split=f[11], loop=f[12], self_index=f[13], early=f[14])
+                        intra_split=f[11], loop=f[12], self_index=f[13], early=f[14],
+                        scan=f[15], more=f[16], scan_grid=f[17])
+    # Which batches the fused scan takes; the other fields of such a plan (form,
+    # nt0, state, split, out, early) describe the operand forms it does not run.
     base = (-1, -1, -1)
+    for T, N, scan in [(8192, 1, 1), (1000, 1, 0), (32768, 2, 1), (8192, 2, 1), (32768, 64, 1)]:
+        assert plans[(T, N, 4, 8) + base]["scan"] == scan, (T, N)
     p = plans[(96, 1, 4, 8) + base]
     assert p["sequential"] == 1
     p = plans[(8192, 1, 4, 8) + base]
@@ -207,6 +212,10 @@ def test_plan_sweep(driver):
             # resident workgroups (2 per CU of 256)
             assert p["state"] % 8 == 0 and p["intra"] % 8 == 0 and p["out"] % 8 == 0, c
             assert p["loop"] == (p["choose"] != 0), c
+            assert p["scan"] == 0 or c[4:6] == (-1, -1), c  # built-in calls only
+            assert (p["scan_grid"] > 0) == (p["scan"] == 1), c
+            # a cut: at most 64 sequences, two launches of at most 512 workgroups
+            assert p["more"] == 0 or (p["scan"] and c[1] <= 64 and 4 * c[3] * p["more"] <= 512), c
             # early output only with the two-segment scan of 8 v-heads, from
             # 30 first-segment chunks on, its grid within the 256 CUs
             assert p["early"] in (0, 64), c
@@ -324,3 +333,20 @@ def test_scan_leaves_short_chains_to_the_operand_forms(driver):
                               (2, 8, 16, 1), (3, 6, 16, 1)]:
         assert _plan(driver, 64 * mean * N - 64 * N, N, 1, hv, -1, -2, -1)["scan"] == 0
         assert _plan(driver, 64 * mean * N - 64 * N, N, 1, hv, -1, -1, -1)["scan"] == scan, (N, hv, mean)
+
+
+def test_batches_of_the_scan_tests_take_it(driver):
+    import test_scan_gpu as scan
+    for name, lens in scan.BATCHES.items():
+        p = _plan(driver, sum(lens), len(lens), 4, 8, -1, -1, -1)
+        assert p["scan"] == 1 and not p["sequential"], name
+        if scan.is_cut(name):
+            chunks = [(n + 63) // 64 for n in lens]
+            length = int(driver([f"seg 8 {p['more']} {' '.join(map(str, chunks))}"])[0])
+            assert p["more"] > 0 and 4 <= length < max(chunks), name
+    for lens in scan.STRESS:
+        p = _plan(driver, sum(lens), len(lens), 4, 8, -1, -1, -1)
+        assert p["scan"] == 1 and p["choose"] == 0, lens
+    # an explicit recurrent_max_len or variant keeps the operand forms
+    for tuning in [(-1, -2, -1), (-1, 64, -1), (0, -1, -1), (1, -1, -1), (2, -1, -1), (3, -1, -1)]:
+        assert _plan(driver, 8192, 1, 4, 8, *tuning)["scan"] == 0

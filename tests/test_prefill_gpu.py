@@ -47,8 +47,9 @@ def to_dev(inp, dev, cu_dtype=torch.int64):
     return d
 
 
-# "auto": the built-in per-sequence routing (short sequences token by token);
-# "chunked": every sequence through the chunk-64 pipeline.
+# "auto": the built-in routing (short batches token by token or in blocks, most
+# others through the fused scan); "chunked": every sequence through the
+# operand-form pipeline.
 ROUTES = {"auto": -1, "chunked": -2}
 
 
@@ -197,8 +198,9 @@ def test_prefill_forms_reference_and_edge_cases(cuda_device, form):
                                   [256] * 4, [384] * 8, [150] * 12, [100, 700], [800, 64, 64],
                                   [128] * 16, [768] * 12])
 def test_prefill_built_in_form_choice(cuda_device, lens):
-    # The built-in choice is bit-identical to the form the rule names, and
-    # the flag the index kernel leaves in the workspace is that form.
+    # The operand forms' own choice (an explicit recurrent_max_len) is
+    # bit-identical to the form the rule names, and the flag the index kernel
+    # leaves in the workspace is that form.
     from gdn_amd import prefill
     print(f"prefill form choice lens={len(lens)}x{lens[0]}.. expect {form_rule(lens)}", flush=True)
     inp = O.make_prefill_inputs(lens, seed=21)
@@ -581,8 +583,9 @@ def _stream(dev):
 # half of the chunks runs beside the first from a zero state and from the
 # identity, and the second segment's output and new_state then apply the
 # first half's final state.
-# variant 3 forces it (one sequence of >= 2 chunks), 2 forbids it; the built-in
-# choice takes it from 9 chunks on.
+# variant 3 forces it (one sequence of >= 2 chunks), 2 forbids it; the operand
+# forms' own choice (an explicit recurrent_max_len) takes it from 9 chunks on.
+# A built-in call of that length is the fused scan's (tests/test_scan_gpu.py).
 SPLIT, CHAIN = 3, 2
 
 
@@ -605,7 +608,7 @@ def test_prefill_two_segment_scan(cuda_device, L, with_state, slow):
 
 
 @pytest.mark.parametrize("L, expect", [(512, CHAIN), (577, SPLIT), (1024, SPLIT), (8192, SPLIT)])
-def test_prefill_two_segment_built_in_choice(cuda_device, L, expect):
+def test_prefill_two_segment_operand_forms_choice(cuda_device, L, expect):
     print(f"prefill two-segment choice L={L} expect variant {expect}", flush=True)
     inp = O.make_prefill_inputs([L], seed=41, with_state=True)
     d = to_dev(inp, cuda_device)

@@ -1,8 +1,9 @@
 """The fused scan (csrc/gdn_scan.hip), which the built-in prefill takes for
 most batches: lengths at the edges of its tiles, segments and launches, head
-layouts, states, and batches it must split or leave whole, against the CPU
-oracle at the operator tolerance; and the matrix-instruction chains of its
-object file on the CPU.
+layouts, states, extreme inputs, and batches it must cut or leave whole, against
+the CPU oracle at the operator tolerance; that these batches take it, from the
+host's plan (tests/test_host_sanitize.py) and from what the device left in the
+workspace; and the matrix-instruction chains of its object file on the CPU.
 """
 
 import os
@@ -11,15 +12,16 @@ import numpy as np
 import pytest
 import torch
 
-from conftest import assert_output_close, assert_state_close
+from conftest import assert_output_close, assert_output_close_to_row_max, assert_state_close
 from oracle import gdn_oracle as O
 from test_mfma_chains import BUILD, _disassemble, _functions, _need_tools, _violations
 
 from gdn_amd import prefill  # noqa: E402
 
 # lens -> what the batch exercises.  One sequence of 97..704 tokens (at most
-# 11 chunks) and of 2049 on runs the scan at 8 v-heads; from about 24 chunks a
-# lone sequence is cut into segments of at least 4 chunks.
+# 11 chunks) and of 2049 on runs the scan at 8 v-heads, the latter cut into
+# segments of at least 4 chunks; the batches with "cut" or "long" in their name
+# are cut.
 BATCHES = {
     "one_partial": [97],
     "one_full": [128],
@@ -29,6 +31,8 @@ BATCHES = {
     "cut_exact": [2560],                # 40 chunks: eight segments of 5
     "cut_many": [8191],
     "two_cut": [4100, 2111],
+    "three_cut": [1280] * 3,            # a workgroup a compute unit: segments of 7
+    "four_cut_long": [8191] * 4,        # two workgroups a compute unit
     "four_cut": [4096, 4033, 64, 2950],
     "ragged_cut": [6, 49, 294, 1800, 2040, 61],
     "long_among_ones": [3000] + [1] * 63,   # 64 sequences, the most that are cut
@@ -38,9 +42,13 @@ BATCHES = {
 }
 
 
+def is_cut(name):
+    return "cut" in name or "long" in name
+
+
 def _words(ws, T, N):
-    """(chunks, path flag, segment length or operand form) that a batch of N > 1
-    sequences left in its workspace, after the offsets of its sequences."""
+    """(chunks, path flag, segment length) that a batch left in its workspace,
+    after the offsets of its sequences (one sequence: the length alone)."""
     at = (O.max_chunks(T, N) * 16 + 255) // 256 * 256 + N * 4
     return ws[at:at + 12].cpu().numpy().view(np.int32).tolist()
 
@@ -68,9 +76,20 @@ def test_scan_matches_oracle(cuda_device, name):
     inp = O.make_prefill_inputs(lens, seed=300 + len(name), with_state=len(name) % 2 == 0,
                                 slow_decay_heads=(0, 7) if "cut" in name else ())
     o_ref, s_ref = O.prefill_seq_c(**inp)
-    o, s = _run(inp, cuda_device)
+    T, N = sum(lens), len(lens)
+    ws = prefill.alloc_workspace(T, N, cuda_device)
+    ws.fill_(0xFF)  # nothing in it needs to hold anything
+    o, s = _run(inp, cuda_device, workspace=ws)
     assert_output_close(o, o_ref)
     assert_state_close(s, s_ref)
+    _, sequential, length = _words(ws, T, N)
+    if N > 1:
+        assert sequential == 0
+    if is_cut(name):
+        assert 4 <= length < max(lens) // 64, length
+    # a second pass gives the same bits
+    o2, s2 = _run(inp, cuda_device)
+    assert np.array_equal(o, o2) and np.array_equal(s, s2)
 
 
 @pytest.mark.gpu
@@ -97,6 +116,70 @@ def test_scan_cut_partial_batch(cuda_device, T, cu):
     o, s = _run(inp, cuda_device)
     assert not o[:cu[0]].any() and not o[cu[-1]:].any()
     assert_output_close(o, o_ref)
+    assert_state_close(s, s_ref)
+
+
+# The stress inputs of the operand forms' tests (tests/test_prefill_gpu.py) through
+# the scan: whole, cut, and cut beside a short sequence.
+STRESS = [[200, 64, 130], [2600], [2600, 700], [1300, 1290, 40]]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens", STRESS, ids=lambda x: "_".join(map(str, x)))
+def test_scan_extreme_gates(cuda_device, lens):
+    # Per-head gates around softplus' threshold (x > 20), beta saturated at 0
+    # and 1, decays ~1 (segment maps near the identity) and so fast that exp(G)
+    # underflows inside a chunk.
+    print(f"scan extreme gates lens={lens}", flush=True)
+    T = sum(lens)
+    inp = O.make_prefill_inputs(lens, seed=361)
+    rng = np.random.default_rng(361)
+    a_h = np.array([30.0, -30.0, 20.0, 0.0, 19.5, -5.0, 5.0, 1.0], np.float32)
+    b_h = np.array([-40.0, 40.0, 0.0, 8.0, -8.0, 1.0, -1.0, 0.0], np.float32)
+    inp["a"][:] = O.bf16_round(a_h[None, :] + rng.normal(0, 0.5, (T, 8)).astype(np.float32))
+    inp["b"][:] = O.bf16_round(b_h[None, :] + rng.normal(0, 0.5, (T, 8)).astype(np.float32))
+    inp["A_log"][:] = np.array([-10.0, 2.7, 0.0, -20.0, 1.0, 0.5, 0.1, 2.0], np.float32)
+    o_ref, s_ref = O.prefill_seq_c(**inp)
+    o, s = _run(inp, cuda_device)
+    assert_output_close(o, o_ref)
+    assert_state_close(s, s_ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens", STRESS, ids=lambda x: "_".join(map(str, x)))
+def test_scan_operand_magnitudes(cuda_device, lens):
+    # Keys and values far from unit size, per head (q/k head 0 keys x 1e-3, head 1
+    # x 0.05; v-heads 0-1 values x 1e4, 2-3 x 1e-4), each head against its own
+    # magnitude.
+    print(f"scan operand magnitudes lens={lens}", flush=True)
+    inp = O.make_prefill_inputs(lens, seed=362, slow_decay_heads=(7,))
+    inp["k"] = O.bf16_round(inp["k"] * np.array([1e-3, 0.05, 1.0, 1.0], np.float32)[None, :, None])
+    vs = np.array([1e4, 1e4, 1e-4, 1e-4, 1.0, 1.0, 1.0, 1.0], np.float32)
+    inp["v"] = O.bf16_round(inp["v"] * vs[None, :, None])
+    inp["state"] = (inp["state"] * vs[None, :, None, None]).astype(np.float32)
+    o_ref, s_ref = O.prefill_seq_c(**inp)
+    o, s = _run(inp, cuda_device)
+    for h in range(8):
+        m = max(float(np.abs(o_ref[:, h]).max()), 1e-30)
+        assert_output_close(o[:, h] / m, o_ref[:, h] / m, what=f"output head {h}")
+        assert_state_close(s[:, h], s_ref[:, h], what=f"state head {h}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("noise", [0.0, 0.1])
+def test_scan_all_same(cuda_device, noise):
+    # The reference's adversarial family: equal keys, the state growing to ~1e27
+    # within two chunks.  Single bf16 operands of the output products: the row
+    # bound of conftest.py where the growth is uneven.
+    lens = [100] if noise == 0.0 else [70, 48, 64]
+    print(f"scan all_same lens={lens} noise={noise}", flush=True)
+    inp = O.make_all_same_inputs(lens, noise=noise, seed=3)
+    o_ref, s_ref = O.prefill_seq_c(**inp)
+    o, s = _run(inp, cuda_device)
+    if noise == 0.0:
+        assert_output_close(o, o_ref)
+    else:
+        assert_output_close_to_row_max(o, o_ref)
     assert_state_close(s, s_ref)
 
 

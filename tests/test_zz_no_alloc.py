@@ -23,7 +23,7 @@ pytestmark = pytest.mark.gpu
 
 from gdn_amd import _lib  # noqa: E402
 
-# (lengths, seed): one sequence long enough for the two-segment scan, then a
+# (lengths, seed): one sequence long enough to be cut into segments, then a
 # smaller packed batch (device-built chunk index), then a large one again.
 CALLS = [
     ([3000], 90),
