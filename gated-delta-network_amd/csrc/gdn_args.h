@@ -53,7 +53,8 @@ int check_decode_args(const gdn_bf16 *q, const gdn_bf16 *k, const gdn_bf16 *v, c
 // tiling, 0 .. kNumRecTilings - 1 a token-by-token tiling, kNumRecTilings the
 // 16-token block kernel.  `variant` -1 is the built-in
 // choice (token by token or blocks by the cost models, at B = 64: 4 tokens
-// 18.8 vs 19.5 us, 8 tokens 26.3 vs 19.9 us, 16 tokens 41.2 vs 20.6 us);
+// 15.9 vs 16.0 us, 5 tokens 17.7 vs 16.2, 8 tokens 21.9 vs 16.3, 16 tokens 35.9
+// vs 16.5; within 0.3 us of the faster kernel for B = 1..256 rows of 2..16);
 // the block kernel reads q, k and v rows with 16-byte loads, so it is never
 // chosen for, and refuses, rows that are not 16-byte aligned.
 constexpr int kDecodeStep = -2;
@@ -110,7 +111,7 @@ long long max_chunks(long long T, long long N);
 PrefillLayout prefill_layout(int T, int N, const Heads &H);
 
 // Arguments of a prefill call: counts, pointers, scale, alignment, the tuning
-// choices (variant -1..3, rec_max >= -2, rec_variant -1..num_rec_variants-1),
+// choices (variant -1..4, rec_max >= -2, rec_variant -1..num_rec_variants-1),
 // the workspace (none needed for N == 0) and every forbidden overlap.  Fills
 // *L with the workspace layout.  GDN_OK or an error.
 int check_prefill_args(const gdn_bf16 *q, const gdn_bf16 *k, const gdn_bf16 *v, const float *state,
@@ -136,12 +137,14 @@ int check_prefill_args(const gdn_bf16 *q, const gdn_bf16 *k, const gdn_bf16 *v, 
 constexpr int kRecurrentMaxLen = 96;
 
 // Two-segment scan of one sequence (state kernel, SplitScan): three groups of
-// 8 workgroups per v-head, one per CU, so it needs 24 H.v <= 256; the built-in
-// choice takes it from kSplitMinChunks chunks on (MI355X, graph replay, one
+// 8 workgroups per v-head, one per CU, so it needs 24 H.v <= 256; the operand
+// forms take it from kSplitMinChunks chunks on (MI355X, graph replay, one
 // chain vs two segments: 28.3 vs 28.4 us at 8 chunks, 30.3 vs 29.5 at 9, 39.3
 // vs 35.3 at 16, 53.3 vs 43.9 at 32, 64.5 vs 53.1 at 40).  Variants: 0 / -1
-// built in, 2 never (one chain), 3 always (one sequence of at least two
-// chunks).
+// by that rule, 2 never (one chain), 3 always (one sequence of at least two
+// chunks).  A built-in call runs the two segments up to 256 / H.v chunks, where
+// the fused scan takes over (scan_wins); longer ones, and the early output, are
+// reached through an explicit variant or recurrent_max_len only.
 constexpr int kSplitMinChunks = 9;
 
 // Chunks that the longest sequence could have, by (T, N) alone, from which on a
@@ -181,9 +184,11 @@ struct PrefillPlan {
   int form;         // per-chunk operands: 0 WY, 1 T, -1 the index kernel's rule
   bool scan;        // the chunks through the fused scan (gdn_scan.hip) instead of the
                     // operand-form pipeline the fields below describe.  The choice
-                    // between sequential and chunks stays the operand forms': the
-                    // sequential kernels are the more precise ones, so no batch
-                    // leaves them for the scan's sake
+                    // between sequential and chunks stays the operand forms': with a
+                    // carried state the sequential kernels are the more precise ones
+                    // (q S takes it in f32 or as hi + lo, the scan as one bf16:
+                    // output error against float64 2.3e-3, the scan's 2.9e-3), so
+                    // no batch leaves them for the scan's sake
   int scan_more;    // most segments beyond the sequences' first ones (0: none is cut)
   long long scan_grid;  // fused scan: workgroups of the first segments' output; fewer
                     // than the N * H.v * 4 units they loop over when the device makes

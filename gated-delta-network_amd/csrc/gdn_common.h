@@ -30,7 +30,10 @@ struct Heads {
 // per token and state traffic per group (refit after the kernel's state
 // accesses went non-temporal and its tiling was re-swept: 86 shapes N =
 // 1..256, L = 1..512, rms error 6 %, largest 21 % at 256 one-token sequences,
-// where the state traffic binds).
+// where the state traffic binds).  Not refitted since the tilings of rec_tiling
+// (gdn_args.h): it reads 8 % high at B = 64, T = 4 (17.2 us for 15.9), as the
+// block model does (18.9 for 16.0), and the choice between them still falls on
+// the faster kernel.
 __host__ __device__ inline float cost_by_token(float L, float T, float hv, float g) {
   return 3.56f + 0.216f * L + 0.00297f * T * hv + 0.0131f * g;
 }
@@ -86,7 +89,9 @@ __host__ __device__ inline float cost_by_chunks(float L, float nt, float hv, flo
                              t_form_wins(nt, ceilf(L / 64.0f), state_units(N, hv)));
 }
 
-// What a path choice made on the device costs (graph replay, MI355X): the
+// What a path choice made on the device costs (graph replay, MI355X, the
+// operand forms' launches; the fused scan's idle grids cost as much, 55 us a
+// call of 256 x 1 tokens either way): the
 // index kernel and the chunk kernels returning at once when the sequential
 // path wins (~9 us over the sequential kernel alone), the sequential kernel
 // returning at once when the chunks win (~5 us).  The device prefers the

@@ -34,6 +34,10 @@
 //               (after a two-segment scan of one sequence, 3b: with the
 //               second segment's output in the same launch).
 //
+// Built-in calls run this pipeline for a few sequences of middling length only
+// (scan_wins in gdn_args.cpp); most go through the fused scan (gdn_scan.hip), and
+// the rest of it is reached through the tuning arguments.
+//
 // Two forms of the state-independent per-chunk operands, chosen per batch:
 //   WY form: the intra kernel forms w and u (and K^T fragments); a state step
 //            is v_new = u - w S, then the update: two LDS exchanges.  The

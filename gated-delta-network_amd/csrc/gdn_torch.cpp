@@ -6,7 +6,7 @@
 // start.
 //
 // The checks and the unpacking of eleven tensors took the Python path ~6 us a
-// call, more than a small decode step takes on the GPU (B = 1: 8.6 -> 4.0 us
+// call, more than a small decode step takes on the GPU (B = 1: 8.5 -> 4.3 us
 // per step back to back).
 #include <Python.h>
 

@@ -185,9 +185,10 @@ def kernel(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output, new_
     zeros); scale float, 0-d tensor or
     None; output [T,8,128] bf16; new_state [N,8,128,128] f32 (may be state).
     ``variant`` picks the form of the per-chunk operands
-    (gdn_prefill_fwd_variant): 0 WY, 1 T, -1 the built-in choice; 2 WY with
+    (gdn_prefill_fwd_variant): -1 the built-in choice, for most batches the
+    fused scan; 0 WY, 1 T, 2 WY with
     one serial chain per sequence, 3 WY with the two-segment scan of a single
-    sequence (0 and -1 take it from 9 chunks on), 4 as 3 with the state
+    sequence (0 takes it from 9 chunks on), 4 as 3 with the state
     launch's early output of the first half stopped after one chunk per
     workgroup (the output launch then computes the rest: a test of that
     path).  ``workspace``: a caller-owned uint8
@@ -195,7 +196,7 @@ def kernel(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output, new_
     ``recurrent_max_len``: a batch whose longest sequence has at most this
     many tokens runs through the sequential kernel instead of the chunks (-1
     built-in: token by token, in 16-token blocks or chunks by fitted cost
-    models; -2 never);
+    models; -2 never); any value but -1 keeps the chunks to the operand forms;
     ``recurrent_variant``: the sequential kernel (gdn_prefill_fwd_tuned):
     0..9 a token-by-token row tiling, 10 the 16-token block kernel.
     """

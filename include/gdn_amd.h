@@ -192,9 +192,12 @@ int gdn_prefill_status(const void *workspace, int total_tokens, int num_seqs, in
  * host picks the faster sequential kind at the mean length and, unless the
  * chunks win for any longest sequence, the device compares cost models of
  * it and of the chunks from the longest sequence, the chunk count, T and N
- * (fitted on MI355X: many short-to-medium sequences go in blocks, e.g. 64 x
- * 256 tokens 115 us vs 171 us through the chunks).  Results agree within the
- * stated tolerance either way (the reference measured the same crossover
+ * (fitted on MI355X: many short-to-medium sequences go in blocks).  The chunks
+ * run as a fused scan that computes the output beside the recurrence and cuts
+ * long sequences into segments (csrc/gdn_scan.hip), except for a few sequences
+ * of middling length, which keep the operand forms of gdn_prefill_fwd_variant
+ * (scan_wins in csrc/gdn_args.cpp).  Results agree within the stated tolerance
+ * either way (the reference measured the same crossover
  * between its sequential scan and chunked kernels,
  * OPTIMIZATION_LOG.md:79,170-184).
  */
@@ -212,7 +215,9 @@ int gdn_prefill_fwd(const gdn_bf16 *q, const gdn_bf16 *k, const gdn_bf16 *v,
  * shortest chain), 1 = T form (the intra kernel stores only (I+A)^-1; each
  * state step forms beta V - beta e^G K S from the inputs: less memory
  * traffic, one more exchange per step), -1 = the built-in choice (what
- * gdn_prefill_fwd uses, decided on the device: the T form for batches of at
+ * gdn_prefill_fwd uses: the fused scan for most batches; for the others, and
+ * under an explicit recurrent_max_len of gdn_prefill_fwd_tuned, one of the two
+ * forms, decided on the device: the T form for batches of at
  * least 144 chunks with more than three times the chunks of their longest
  * sequence, or of at least 384 with at least 1.5 times, and for batches of
  * at most 768 state units -- sequence x v-head x 16-column block -- whose
@@ -222,7 +227,8 @@ int gdn_prefill_fwd(const gdn_bf16 *q, const gdn_bf16 *k, const gdn_bf16 *v,
  * scan for a single sequence of at least two chunks (the second half of the
  * chunks runs beside the first from a zero state and from the identity, and
  * one more launch applies the first half's final state: half the serial
- * chain; 0 and -1 take it from 9 chunks on when 24 x num_v_heads <= 256;
+ * chain; the WY form of 0 and -1 takes it from 9 chunks on when 24 x
+ * num_v_heads <= 256;
  * with 8 v-heads and at least 30 first-half chunks the state launch also
  * computes the first half's output as its chain goes, on the CUs the scan
  * leaves idle), 4 = as 3 with that early output stopped after one chunk per
@@ -249,7 +255,9 @@ int gdn_prefill_fwd_variant(const gdn_bf16 *q, const gdn_bf16 *k, const gdn_bf16
  *                      (-1 built-in)
  *   recurrent_max_len  a batch whose longest sequence has at most this many
  *                      tokens runs through the sequential kernel; -1 =
- *                      built-in, -2 = never (always chunked)
+ *                      built-in, -2 = never (always chunked).  Any value but
+ *                      -1 runs the chunks in the operand forms, never as the
+ *                      fused scan, as does an explicit state_tiling
  *   recurrent_tiling   the sequential kernel, as the variant of
  *                      gdn_decode_multi_fwd (10 = blocks; -1 built-in: token
  *                      by token, or under the built-in path choice the kind
