@@ -125,7 +125,7 @@ constexpr int kMinCut = 16;
 // sequences' first ones (the second launch's grid), and as many workgroups in
 // the first.
 // Of the lengths that cut the longest sequence into eight to three, from the
-// shortest on, one is taken over a shorter one if its estimate is a tenth
+// shortest on, one is taken over a shorter one if its estimate is 7 %
 // lower, and any if it beats the whole sequences.  The shortest that fits the
 // grid is often not the best: as soon as a launch has more workgroups than
 // compute units, its steps take longer, and by more where the v-heads are no
@@ -133,44 +133,49 @@ constexpr int kMinCut = 16;
 // run on different ones, each with its own L2).  us, shortest / best: 3 x 20
 // chunks of 8 v-heads, 4 chunks 53.3 / 7 chunks 45.5; 32 chunks of 10 v-heads, 4
 // chunks 53.2 / 5 chunks 46.2; 2 x 32 of 8, 4 chunks 58.3 / 7 chunks 49.4.
-// Estimates in microseconds, fitted to every length of 1450 batches of N = 1..8
-// equal sequences of 16..128 chunks with 1..64 v-heads and 127 uneven ones of
-// 2..64 sequences.
+// Estimates in microseconds, fitted to the times of every length of 1264 batches of
+// N = 1..8 equal sequences of 16..128 chunks with 1..64 v-heads and 274 uneven
+// ones of 2..64 sequences (its lengths take 0.8 % above the best on average).
 template <class Sum>
 __host__ __device__ inline int segment_choice(int longest, int max_more, int hv, Sum sum) {
   if (longest < kMinCut) return 0;
   const float cus = static_cast<float>(hv) * (4.0f / 256.0f);  // CUs of one slot's workgroups
   const bool xcds = hv % 8 == 0;
   // step time relative to a CU of its own, w workgroups a CU
-  auto share = [](float w) { return w <= 1.0f ? 1.0f : 1.15f + 0.4f * (w - 1.0f); };
-  const float work = 1.05f * cus * static_cast<float>(sum([](int n) { return n; }));
+  auto share = [](float w) { return w <= 1.0f ? 1.0f : 1.12f + 0.46f * (w - 1.0f); };
+  const int total = sum([](int n) { return n; });
+  const float work = 1.15f * cus * static_cast<float>(total);
   const float w0 = fminf(cus * static_cast<float>(sum([=](int n) { return 2 * n > longest ? 1 : 0; })), 2.0f);
-  const float whole = fmaxf(1.3f * share(w0) * static_cast<float>(longest) + (w0 > 1.0f ? 4.0f : 0.0f), work);
+  const float whole = fmaxf(1.3f * share(w0) * static_cast<float>(longest) + (w0 > 1.0f ? 2.75f : 0.0f), work);
   int best_len = 0;
   float best = 0.0f;
   for (int parts = 8; parts >= 3; --parts) {
     int len = (longest + parts - 1) / parts;
     len = len < kMinSegment ? kMinSegment : len;
     if (2 * len >= longest) continue;
-    // segments beyond the first, maps, first segments that are full: at most
-    // eight of each a sequence, of at most 64
+    // segments beyond the first ((n - 1) / len, at most seven), maps, first
+    // segments that are full, of at most 64 sequences
     const int counts = sum([=](int n) {
-      const int more = n > len ? (n - 1) / len : 0;
+      int more = 0;
+      for (int p = 1; p < 8; ++p) more += n > p * len ? 1 : 0;
       return more | (more > 1 ? more - 1 : 0) << 10 | (n >= len ? 1 : 0) << 20;
     });
     const int second = counts & 1023, mids = (counts >> 10) & 1023, first = (counts >> 20) + mids;
     if (first > max_more || second > max_more) continue;
-    const float w = cus * static_cast<float>(first > second ? first : second);
-    const float step = 2.9f * share(w) * (w > 1.0f && !xcds ? 1.5f : 1.0f);
+    // chain steps of the two launches, in workgroups of len steps a CU
+    const int steps1 = sum([=](int n) { return n < len ? n : len; });
+    const int most = steps1 + mids * len > total - steps1 ? steps1 + mids * len : total - steps1;
+    const float w = cus * static_cast<float>(most) / static_cast<float>(len);
+    const float step = 2.7f * share(w) * (w > 1.0f && !xcds ? 1.7f : 1.0f);
     const float chain = step * static_cast<float>(len) +
-                        1.5f * static_cast<float>((longest + len - 1) / len - 2) +
-                        (w > 1.0f ? 12.0f : 4.0f) + (xcds ? 0.0f : 3.0f * w);
-    const float est = fmaxf(chain, work + 1.2f * cus * static_cast<float>(mids * len) + 8.0f);
-    if (best_len == 0 || est < 0.9f * best) {
+                        0.75f * static_cast<float>((longest + len - 1) / len - 2) +
+                        (w > 1.0f ? 9.5f : 4.0f) + (xcds ? 0.0f : 6.0f * w);
+    const float est = fmaxf(chain, work + 1.3f * cus * static_cast<float>(mids * len) + 8.0f);
+    if (best_len == 0 || est < 0.93f * best) {
       best = est;
       best_len = len;
     }
-    if (w <= 1.0f) break;  // a longer segment only has fewer workgroups yet
+    if (w <= 1.0f) break;  // a longer one only lengthens the chains
   }
   return best_len != 0 && best < whole ? best_len : 0;
 }
