@@ -32,7 +32,7 @@
 //
 // Measured against the operand-form pipeline (us per call, states given):
 // 64x256 161 -> 93, 16x1024 135 -> 74, 8x2048 133 -> 79, 2x4096 94 -> 70,
-// 4x8192 252 -> 195, 1x8192 110 -> 81, 1x512 27 -> 24; 1x1024 31 -> 35.
+// 4x8192 252 -> 187, 1x8192 110 -> 81, 1x512 27 -> 24; 1x1024 31 -> 35.
 #include "gdn_chunk.h"
 #include "gdn_device.h"
 #include "gdn_host.h"
